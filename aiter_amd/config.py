@@ -80,6 +80,32 @@ def merge_csvs(files: list[str], keys: list[str], result_cols=("kernelName",)) -
     return df
 
 
+class TunedRow(dict):
+    """A tuned row with the row count it serves a call as: ``rows`` is the
+    (padded) M whose entry was found."""
+
+    rows: int = 0
+
+
+def tuned_row(cfg: dict, m: int, rows: int, env_name: str) -> TunedRow:
+    """``cfg`` of a lookup at M = ``m`` that matched the entry for ``rows``.
+    An entry from the caller's own CSV list serves the call as if tuned for it."""
+    row = TunedRow(cfg)
+    row.rows = m if os.environ.get(env_name) else rows
+    return row
+
+
+def row_kernel(row: TunedRow, m: int) -> str:
+    """The row's kernel name as the library takes it for ``m`` rows.  From 64
+    rows on, a shipped row tuned at 1.25 times the rows or more (the
+    power-of-two padding of the lookup) names a tile that may leave a good part
+    of itself empty: "~name" lets the library's time model replace it (bf16 1200 x
+    4096 x 4096, tuned at 2048 rows: 51.9 us by the row, 43.1 by the model's
+    160x128 tile; A4W4 2500 x 7168 x 2048 32.2 and 28.2)."""
+    name = str(row.get("kernelName", "") or "")
+    return "~" + name if name and row.rows > 64 and row.rows >= 1.25 * m else name
+
+
 def load_tuned(env_name: str, default: str, keys: list[str]) -> dict:
     df = merge_csvs(config_files(env_name, default), keys)
     if not len(df):

@@ -15,6 +15,7 @@
 #include <string>
 #include <vector>
 
+#include "gemm_cost.h"
 #include "gemm_registry.h"
 #include "out_quant.h"
 
@@ -53,6 +54,14 @@ std::vector<Instance>& registry() {
         b.part_rest();
         b.part_direct();
         b.part_late();
+        b.part_mid();
+        for (auto& in : reg) {
+            std::string nm = in.name;
+            const size_t f32 = nm.find("_f32");
+            if (f32 != std::string::npos) nm.erase(f32, 4);
+            for (auto& c : kGemmCosts)
+                if (nm == c.name) in.cost = &c;
+        }
     });
     return reg;
 }
@@ -73,10 +82,11 @@ bool variant_ok(const Instance& in, Family f, const Variant& v) {
 }
 
 // Split-K factor for a skinny launch: split only when the 16-column blocks
-// cannot cover the CUs, keeping >= 32 k-steps (8 per wave) per split.
-int skinny_splits(int n_blocks, int k_steps, int cus) {
+// cannot cover the CUs, keeping at least `per_split` k-steps (32: 8 per wave)
+// per split.
+int skinny_splits(int n_blocks, int k_steps, int cus, int per_split = 32) {
     int s = 1;
-    while (n_blocks * s < cus && k_steps / (s * 2) >= 32) s *= 2;
+    while (n_blocks * s < cus && k_steps / (s * 2) >= per_split) s *= 2;
     return s;
 }
 
@@ -88,43 +98,138 @@ int tile_splits(int tiles, int stages, int cus) {
     return s;
 }
 
-// Heuristic choice among tile instances (reference heuristic idea:
-// csrc/py_itfs_cu/asm_gemm_a4w4.cu:81-152 — fewest rounds of tiles over the
-// CUs, then higher tile compute/memory ratio).
-const Instance* heuristic(Family f, const Variant& v, int M, int N, int K, int cus, int* splits) {
+// What the time model may choose for a call: batch > 1 and fused epilogues run
+// one-tile-per-workgroup kernels only.
+struct ModelScope {
+    int batch = 1;
+    bool persistent = true;   // persistent tiles allowed (no bias, batch or fused epilogue)
+};
+
+// Instances with a modelled time, per family and variant.
+const std::vector<const Instance*>& modelled(Family f, const Variant& v) {
+    static std::vector<const Instance*> lists[3][8];
+    static std::once_flag once;
+    std::call_once(once, [] {
+        for (auto& in : registry())
+            if (in.cost && !(in.skinny && in.split))
+                lists[in.fam][in.var.a_pre * 4 + in.var.b_pre * 2 + in.var.out_f32].push_back(&in);
+    });
+    return lists[f][v.a_pre * 4 + v.b_pre * 2 + v.out_f32];
+}
+
+// Modelled time of instance `in` with `splits` K splits, us (gemm_cost.h).
+float model_us(const Instance& in, int M, int N, int K, int splits, int batch, int cus) {
+    const GemmCost& c = *in.cost;
+    const bool mx = in.fam != kA16W16;
+    const int nst = K / (mx ? 256 : 64);
+    const int stages = (nst + splits - 1) / splits;
+    const int64_t tm = in.skinny ? 1 : (M + in.bm - 1) / in.bm, tn = (N + in.bn - 1) / in.bn;
+    const int64_t per_cu = (tm * tn * splits * batch + cus - 1) / cus;
+    float t;
+    if (in.skinny) {
+        const float rounds = (float)((per_cu + 3) / 4);
+        t = stages * std::max(c.stage * rounds, c.shared * per_cu) + c.wg * rounds;
+    } else {
+        t = per_cu * (stages * c.stage + c.wg);
+    }
+    const float mb = 1e-6f * batch;
+    const float abytes = mb * M * K * (in.fam == kA8W4 ? 1.0f : mx ? 0.5f : 2.0f);
+    const float bbytes = mb * N * K * (mx ? 0.53f : 2.0f), dbytes = mb * M * N * 2.0f;
+    t = std::max(t, (abytes + bbytes + dbytes) / 6.6f);
+    // a stage holds 128 bytes of a row (256 of an e4m3 row)
+    const float sbytes = mb * nst * 128.0f;
+    t = std::max(t, (sbytes * (in.fam == kA8W4 ? 2 : 1) * M * tn + sbytes * N * tm) / 15.0f);
+    if (splits > 1) t += 0.22f * (dbytes + 4.0f * dbytes * splits);
+    return c.call + t;
+}
+
+// K splits that a split tile instance runs for a request of `want` (0: the
+// launcher's own choice)
+int tile_split_count(const Instance& in, int M, int N, int K, int cus, int want) {
+    const int nst = K / (in.fam == kA16W16 ? 64 : 256);
+    const int tiles = ((M + in.bm - 1) / in.bm) * ((N + in.bn - 1) / in.bn);
+    const int sp = std::max(1, std::min(want > 0 ? want : tile_splits(tiles, nst, cus), nst));
+    const int per = (nst + sp - 1) / sp;
+    return (nst + per - 1) / per;
+}
+
+// Skinny kernel for M <= 32: 32-column workgroups when they cover 3/4 of the
+// CUs (above 16 rows always: each A fragment then serves two B blocks, whose
+// traffic is the larger part there; up to 16 rows only while they fit one
+// round, at N = 14336 two rounds of them measured 25.0 us against 21.2 in
+// bf16), else 16-column ones, unless only the 32-column form has its operands
+// copied through LDS (MXFP8: 6.3 against 8.8 us at 24 x 1088 x 7168).  K is
+// split only without an LDS form and from K = 16384 (MX) or 8192 (bf16) on: the
+// fill and finish launches cost 3 us (bf16 24 x 3072 x 6144 13.4 unsplit, 24.9
+// split; 1 x 256 x 7168 6.1 / 8.5; A4W4 1 x 1536 x 12288 5.4 / 8.2; preshuffled
+// bf16 1 x 1536 x 12288 20.3 / 14.0).
+const Instance* skinny_rule(Family f, const Variant& v, int M, int N, int K, int cus, int* splits) {
+    const int bm = M <= 16 ? 16 : 32;
+    auto pick = [&](int bn, bool split) {
+        const Instance* got = nullptr;
+        for (auto& in : registry())
+            if (in.skinny && variant_ok(in, f, v) && in.bm == bm && in.bn == bn && in.split == split &&
+                (!got || in.rank > got->rank))
+                got = &in;
+        return got;
+    };
+    const Instance *n16 = pick(16, false), *n32 = pick(32, false);
+    const int blk32 = (N + 31) / 32;
     *splits = 1;
-    const int ksteps = K / (f == kA16W16 ? 32 : 128);
-    if (M <= 32) {
-        const int mf = M <= 16 ? 1 : 2;
-        const int nblk = (N + 15) / 16;
-        const int s = skinny_splits(nblk, ksteps, cus);
-        // 32-column workgroups when M > 8 and they still cover ~3/4 of the
-        // CUs: each A fragment then serves two B blocks (A's L2 traffic per
-        // B byte halves); measured 4.3 -> 4.0 us at M=16 and 5.4 -> 4.4 us at
-        // M=32 for N=7168, K=2048, and no gain at M=1
-        auto pick = [&](int bn, bool split) {
-            const Instance* got = nullptr;
-            for (auto& in : registry())
-                if (in.skinny && variant_ok(in, f, v) && in.bm == 16 * mf && in.bn == bn && in.split == split &&
-                    (!got || in.rank > got->rank))
-                    got = &in;
-            return got;
-        };
-        if (M > 8 && s == 1 && (N + 31) / 32 * 4 >= cus * 3)
-            if (const Instance* in = pick(32, false)) return in;
-        if (const Instance* in = pick(16, s > 1)) {
+    if (n32 && (!n16 || (blk32 * 4 >= cus * 3 && (M > 16 || blk32 <= cus)) || (M > 16 && n32->rank > n16->rank)))
+        return n32;
+    const int s = skinny_splits((N + 15) / 16, K / (f == kA16W16 ? 32 : 128), cus, f == kA16W16 ? 128 : 64);
+    if (s > 1 && n16 && n16->rank == 0)
+        if (const Instance* in = pick(16, true)) {
             *splits = s;
             return in;
         }
+    return n16;
+}
+
+// The instance that the time model puts 6 % or more below `base` with
+// `base_splits` (else base): the model is off by about that much between
+// neighbouring tiles, and without the margin twice as many shapes ran over 5 %
+// slower than by the simple rule.  *splits: the split count of a split tile (0:
+// base).  Splits that need more than `ws_bytes` of partials are left out.
+const Instance* modelled_choice(const Instance* base, int base_splits, int M, int N, int K, int cus,
+                                const ModelScope& sc, size_t ws_bytes, int* splits) {
+    const int nst = K / (base->fam == kA16W16 ? 64 : 256);
+    const Instance* best = base;
+    float best_us = model_us(*base, M, N, K, base_splits, sc.batch, cus) / 1.06f;
+    *splits = 0;
+    for (const Instance* in : modelled(base->fam, base->var)) {
+        if (in->persistent && !sc.persistent) continue;
+        if (in->skinny && (M > in->bm || M * 2 <= in->bm)) continue;
+        if (!in->split) {
+            const float us = model_us(*in, M, N, K, 1, sc.batch, cus);
+            if (us < best_us) best = in, best_us = us, *splits = 1;
+            continue;
+        }
+        if (sc.batch > 1) continue;
+        for (int want = 2; want <= 8 && nst / want >= 4; want *= 2) {
+            const int sp = tile_split_count(*in, M, N, K, cus, want);
+            if (sp < 2 || (size_t)sp * M * N * sizeof(float) > ws_bytes) continue;
+            const float us = model_us(*in, M, N, K, sp, 1, cus);
+            if (us < best_us) best = in, best_us = us, *splits = sp;
+        }
     }
-    // time ~ rounds of tiles x per-tile time, and a tile's time per K step
-    // grows like BM + BN (operand bytes) while its work grows like BM * BN:
-    // minimise rounds * (BM + BN); on ties the larger tile
+    return best;
+}
+
+// Instance for a shape without a tuned row: the skinny form up to 32 rows;
+// above, the tile with the fewest rounds x (BM + BN) (the reference's idea,
+// csrc/py_itfs_cu/asm_gemm_a4w4.cu:81-152) among the power-of-two tiles, split
+// when it leaves most CUs idle.  *splits: K splits it runs (0: the launcher's
+// own count).
+const Instance* simple_rule(Family f, const Variant& v, int M, int N, int K, int cus, int* splits) {
+    *splits = 1;
+    if (M <= 32)
+        if (const Instance* in = skinny_rule(f, v, M, N, K, cus, splits)) return in;
     const Instance* best = nullptr;
-    long best_cost = 1L << 40;
-    long best_tiles = 0;
+    long best_cost = 1L << 40, best_tiles = 0;
     for (auto& in : registry()) {
-        if (in.skinny || in.persistent || in.split || !variant_ok(in, f, v)) continue;   // tuned tables only
+        if (in.skinny || in.persistent || in.split || !in.by_ref || !variant_ok(in, f, v)) continue;
         const long tiles = (long)((M + in.bm - 1) / in.bm) * ((N + in.bn - 1) / in.bn);
         const long rounds = (tiles + cus - 1) / cus;
         const long cost = rounds * (in.bm + in.bn);
@@ -135,15 +240,13 @@ const Instance* heuristic(Family f, const Variant& v, int M, int N, int K, int c
         }
     }
     // a grid that leaves most CUs idle splits K when the tile has a split form
-    const int nst = K / (f == kA16W16 ? 64 : 256);
-    if (best && best_tiles * 2 <= cus && nst >= 16) {
+    if (best && best_tiles * 2 <= cus && K / (f == kA16W16 ? 64 : 256) >= 16)
         for (auto& in : registry())
             if (!in.skinny && in.split && !in.persistent && in.bm == best->bm && in.bn == best->bn &&
                 variant_ok(in, f, v)) {
-                *splits = 0;   // the launcher picks the split count
+                *splits = 0;
                 return &in;
             }
-    }
     return best;
 }
 
@@ -253,8 +356,8 @@ const Instance* reference_tile_instance(const RefTile& t, Family f, const Varian
         const bool want_split = pass == 0 ? t.split : false;
         if (pass == 1 && !t.split) break;
         for (auto& in : registry())
-            if (!in.skinny && !in.persistent && in.split == want_split && in.bm == t.tm && in.bn == t.tn &&
-                variant_ok(in, f, v))
+            if (!in.skinny && !in.persistent && in.by_ref && in.split == want_split && in.bm == t.tm &&
+                in.bn == t.tn && variant_ok(in, f, v))
                 return &in;
     }
     return nullptr;
@@ -330,6 +433,17 @@ float* workspace(int dev, hipStream_t st, size_t bytes, int slot = 0) {
         if (slot == kCounterSlot) AA_HIP(hipMemsetAsync(w.ptr, 0, bytes, st));
     }
     return w.ptr;
+}
+
+// Partials that a call on `st` may put into the workspace: no limit, but under
+// graph capture what is there already (it cannot grow then).
+size_t workspace_limit(int dev, hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    AA_HIP(hipStreamIsCapturing(st, &cs));
+    if (cs == hipStreamCaptureStatusNone) return ~size_t(0);
+    std::lock_guard<std::mutex> lk(workspace_mutex());
+    auto it = workspace_map().find({dev, st, 0});
+    return it == workspace_map().end() ? 0 : it->second.bytes;
 }
 
 struct GemmCall {
@@ -527,26 +641,57 @@ void run_gemm(const GemmCall& c, hipStream_t stream) {
     AA_CHECK(c.batch >= 1 && c.batch < 65536, "batch must be in [1, 65535]");
     const bool batched = c.batch > 1;   // one-pass, one-tile-per-workgroup kernels only
     int splits = 1;
+    // "~name": the choice of a tuned row for other row counts, which the time
+    // model may replace
+    const char* name = c.kernel_name && c.kernel_name[0] ? c.kernel_name : nullptr;
+    const bool hint = name && name[0] == '~';
+    if (hint) ++name;
     if (c.kernel_id >= 0) {
         inst = find_by_id(c.kernel_id);
         AA_CHECK(inst && variant_ok(*inst, c.fam, c.var), "kernel id ", c.kernel_id, " does not fit this GEMM");
-    } else if (c.kernel_name && c.kernel_name[0]) {
+    } else if (name) {
         bool known = false;
-        inst = resolve_name(c.kernel_name, c.fam, c.var, M, &known);
-        AA_CHECK(known, "unknown kernel name '", c.kernel_name, "'");
-        if (inst) AA_CHECK(variant_ok(*inst, c.fam, c.var), "kernel '", c.kernel_name, "' does not fit this GEMM");
+        inst = resolve_name(name, c.fam, c.var, M, &known);
+        AA_CHECK(known, "unknown kernel name '", name, "'");
+        if (inst) AA_CHECK(variant_ok(*inst, c.fam, c.var), "kernel '", name, "' does not fit this GEMM");
     } else if (c.ref_tile.tm > 0) {
         inst = reference_tile_instance(c.ref_tile, c.fam, c.var, M);
     }
     const int ksteps = (int)(K / (scaled ? 128 : 32));
+    // requested split count (0: the launcher chooses); the model's (0: none)
+    int req_splits = c.split_count > 0 ? c.split_count : (c.log2_split >= 0 ? 1 << std::min(c.log2_split, 16) : 0);
+    int auto_splits = 0;
+    const bool named = inst != nullptr;
     if (!inst) {
-        inst = heuristic(c.fam, c.var, (int)M, (int)N, (int)K, cus, &splits);
+        inst = simple_rule(c.fam, c.var, (int)M, (int)N, (int)K, cus, &auto_splits);
         AA_CHECK(inst, "no kernel instance for this GEMM");
+        if (inst->skinny && inst->split) splits = auto_splits;
     } else if (inst->skinny && inst->split) {
         splits = skinny_splits((int)((N + 15) / 16), ksteps, cus);
     }
-    // requested split count (0: the launcher chooses)
-    const int req_splits = c.split_count > 0 ? c.split_count : (c.log2_split >= 0 ? 1 << std::min(c.log2_split, 16) : 0);
+    if ((hint || (!named && req_splits == 0)) && M > 16 && inst->cost) {
+        ModelScope sc;
+        sc.batch = c.batch;
+        sc.persistent = !batched && !p.bias && !c.epi.kind;
+        const int have = !inst->split || inst->skinny ? splits
+                         : batched                    ? 1
+                                                      : tile_split_count(*inst, (int)M, (int)N, (int)K, cus, req_splits);
+        int sp = 0;
+        const Instance* best =
+            modelled_choice(inst, have, (int)M, (int)N, (int)K, cus, sc, c.scratch ? c.scratch_bytes : ~size_t(0), &sp);
+        if (best != inst && best->split && !c.scratch) {
+            // under graph capture the workspace cannot grow
+            const size_t room = workspace_limit(dev, stream);
+            if ((size_t)sp * M * N * sizeof(float) > room)
+                best = modelled_choice(inst, have, (int)M, (int)N, (int)K, cus, sc, room, &sp);
+        }
+        if (best != inst) {
+            inst = best;
+            auto_splits = sp;
+            req_splits = 0;
+            splits = 1;
+        }
+    }
     if (inst->skinny && inst->split && req_splits > 0) splits = req_splits;
     if (inst->skinny) AA_CHECK(M <= inst->bm, "skinny kernel ", inst->name, " covers M <= ", inst->bm);
     AA_CHECK(!c.capture || (inst->skinny && !inst->split && !inst->stream_k && !batched),
@@ -560,7 +705,7 @@ void run_gemm(const GemmCall& c, hipStream_t stream) {
         if (inst->split) {
             // split-K tile: stages of K over gridDim.y, f32 slices, then a sum
             const int nst = (int)(K / (scaled ? 256 : 64));
-            int sp = req_splits > 0 ? req_splits : tile_splits(tiles, nst, cus);
+            int sp = req_splits > 0 ? req_splits : auto_splits > 0 ? auto_splits : tile_splits(tiles, nst, cus);
             if (batched) sp = 1;
             sp = std::max(1, std::min(sp, nst));
             p.k_steps_per_split = (nst + sp - 1) / sp;
@@ -1174,13 +1319,17 @@ int batched_gemm_bf16_tune(aiter_tensor_t* XQ, aiter_tensor_t* WQ, aiter_tensor_
 }
 
 // ---- library-specific introspection (used by the Python tuner) ----------
-int aiter_amd_num_kernels(void) { return (int)registry().size(); }
+int aiter_amd_num_kernels(void) {
+    int n = 0;
+    for (auto& in : registry()) n += in.listed;
+    return n;
+}
 
 // Writes "id,name,family,skinny,bm,bn,split,a_pre,b_pre,out_f32" for kernel
 // `id` into buf; returns -1 if id is out of range.
 int aiter_amd_kernel_info(int id, char* buf, int buflen) {
     const Instance* in = find_by_id(id);
-    if (!in || !buf || buflen <= 0) return -1;
+    if (!in || !in->listed || !buf || buflen <= 0) return -1;
     static const char* fam[] = {"a4w4", "a8w4", "a16w16"};
     snprintf(buf, buflen, "%d,%s,%s,%d,%d,%d,%d,%d,%d,%d", in->id, in->name.c_str(), fam[in->fam],
              (int)in->skinny, in->bm, in->bn, (int)in->split, (int)in->var.a_pre, (int)in->var.b_pre,

@@ -1,0 +1,121 @@
+// Modelled time of a GEMM launch per kernel instance, the dispatch's rule for
+// shapes that no tuned row covers.
+//
+// What bounds a tile kernel here is its workgroup's own stream of stages (128
+// bytes of every row of its tile: the LDS copies and reads, then the MFMAs), so
+// one workgroup's time is a line in its stages, and a launch takes as many of
+// those as the fullest CU has workgroups:
+//   us = call + max(per_cu * (stages * stage + wg), bytes / 6.6 TB/s, traffic / 15 TB/s)
+// (skinny kernels share a CU four at a time: stages * max(stage * ceil(per_cu / 4),
+// shared * per_cu) + wg * ceil(per_cu / 4) inside the max).  bytes: A, B and
+// out once; traffic: the operands once per tile that reads them.  A split adds
+// its f32 slices at 0.22 us per MB (written, read, summed).
+//
+// The constants are a fit to 8,200 graph-replayed timings under sustained load
+// (977 shapes with 17 to 8192 rows, N 256 to 28672, K 512 to 28672, splits of 2,
+// 4 and 8; weights rotated) on one MI355X.  Against the best instance of each
+// shape the dispatch's choice (modelled_choice(), gemm.hip) is 3.5 % (bf16), 2.5 %
+// (A4W4) and 2 % (A8W4) slower on average; by the simple rule alone it would
+// be 11-12 %, 8 % and 8 %.
+#pragma once
+
+namespace aiter_amd {
+
+struct GemmCost {
+    const char* name;   // instance name; an f32-output form takes its bf16 form's
+    float stage, shared, call, wg;
+};
+
+inline const GemmCost kGemmCosts[] = {
+    {"a4w4_tile_256x256_persist", 1.21, 0, 0.5, 8.37},
+    {"a4w4_tile_256x256", 1.24, 0, 0.5, 9.95},
+    {"a4w4_tile_128x256_persist", 0.726, 0, 1.91, 4.48},
+    {"a4w4_tile_128x256", 0.74, 0, 0.5, 6.54},
+    {"a4w4_tile_256x128", 0.827, 0, 1.15, 5.68},
+    {"a4w4_tile_192x128", 0.712, 0, 1.07, 4.45},
+    {"a4w4_tile_128x128", 0.45, 0, 0.5, 4.17},
+    {"a4w4_tile_96x128", 0.407, 0, 0.891, 3.4},
+    {"a4w4_tile_192x128_splitk", 0.585, 0, 7.73, 0.01},
+    {"a4w4_tile_64x128_splitk", 0.253, 0, 6.68, 0.894},
+    {"a4w4_tile_32x128_splitk", 0.214, 0, 6.02, 1.26},
+    {"a4w4_tile_128x64_splitk", 0.295, 0, 6.9, 0.01},
+    {"a4w4_tile_64x256_splitk", 0.412, 0, 6.52, 1.26},
+    {"a4w4_tile_96x128_splitk", 0.347, 0, 6.69, 0.645},
+    {"a4w4_tile_128x128_splitk", 0.339, 0, 7.58, 0.211},
+    {"a4w4_tile_32x128", 0.265, 0, 2.81, 1.15},
+    {"a4w4_skinny_m32_alds", 0.0526, 0.0491, 3.41, 0.01},
+    {"a4w4_skinny_m32", 0.116, 0.12, 3, 0.0103},
+    {"a4w4_skinny_m32_n32_alds", 0.0755, 0.0739, 3.49, 0.01},
+    {"a4w4_skinny_m32_n32", 0.152, 0.175, 2.06, 0.77},
+    {"a4w4_tile_64x128", 0.319, 0, 1.47, 2.71},
+    {"a4w4_tile_128x64", 0.329, 0, 1.41, 2.8},
+    {"a4w4_tile_64x256", 0.517, 0, 0.54, 4.15},
+    {"a4w4_skinny_m64_n32_alds", 0.106, 0.000198, 3.81, 0.01},
+    {"a4w4_skinny_m64", 0.21, 0.202, 3.03, 0.01},
+    {"a4w4_skinny_m64_n32", 0.208, 0.256, 2.64, 0.344},
+    {"a8w4_tile_128x256_persist", 1.07, 0, 3.22, 4.84},
+    {"a8w4_tile_128x256", 1.12, 0, 0.5, 7.71},
+    {"a8w4_tile_64x256", 0.773, 0, 0.852, 3.73},
+    {"a8w4_tile_64x128", 0.406, 0, 1.25, 2.97},
+    {"a8w4_tile_96x128", 0.65, 0, 0.957, 3.19},
+    {"a8w4_tile_128x128", 0.756, 0, 0.942, 3.74},
+    {"a8w4_tile_128x64", 0.483, 0, 1.55, 2.7},
+    {"a8w4_tile_64x128_splitk", 0.364, 0, 6.82, 0.159},
+    {"a8w4_tile_32x128_splitk", 0.291, 0, 6.6, 0.01},
+    {"a8w4_tile_128x64_splitk", 0.584, 0, 3, 2.79},
+    {"a8w4_tile_64x256_splitk", 0.772, 0, 6.15, 0.01},
+    {"a8w4_tile_96x128_splitk", 0.52, 0, 7.42, 0.01},
+    {"a8w4_tile_128x128_splitk", 0.797, 0, 3.66, 2.13},
+    {"a8w4_skinny_m32_n32_alds", 0.118, 0.12, 3.5, 0.01},
+    {"a8w4_skinny_m32", 0.212, 0.199, 2.18, 0.769},
+    {"a8w4_skinny_m32_n32", 0.129, 0.25, 1.94, 0.885},
+    {"a8w4_tile_32x128", 0.325, 0, 1.53, 2.37},
+    {"a8w4_skinny_m64", 0.338, 0.359, 2.35, 0.837},
+    {"a16w16_tile_256x256_bplain_flat", 1.29, 0, 0.5, 8.24},
+    {"a16w16_tile_128x256_bplain", 0.788, 0, 0.5, 5.65},
+    {"a16w16_tile_160x128_bplain", 0.577, 0, 0.632, 3.41},
+    {"a16w16_tile_256x128_bplain", 0.766, 0, 0.5, 5.75},
+    {"a16w16_tile_128x256_splitk_bplain", 0.811, 0, 5.87, 0.01},
+    {"a16w16_tile_128x128_bplain", 0.453, 0, 0.5, 3.44},
+    {"a16w16_tile_256x128_splitk_bplain", 0.796, 0, 4.88, 0.01},
+    {"a16w16_tile_160x128_splitk_bplain", 0.523, 0, 6.44, 0.01},
+    {"a16w16_tile_64x128_splitk_bplain", 0.279, 0, 6.63, 0.01},
+    {"a16w16_tile_96x128_bplain", 0.245, 0, 6.02, 0.01},
+    {"a16w16_tile_128x64_splitk_bplain", 0.36, 0, 4.01, 1},
+    {"a16w16_tile_128x128_splitk_bplain", 0.487, 0, 5.87, 0.01},
+    {"a16w16_tile_256x256_bplain", 1.59, 0, 3.95, 4.84},
+    {"a16w16_tile_96x128_splitk_bplain", 0.345, 0, 6.64, 0.01},
+    {"a16w16_tile_64x64_splitk_bplain", 0.237, 0, 5.99, 0.01},
+    {"a16w16_skinny_m32_bplain_lds", 0.0994, 0.105, 0.5, 1.23},
+    {"a16w16_tile_128x64_bplain", 0.283, 0, 0.746, 2.8},
+    {"a16w16_tile_64x128_bplain", 0.263, 0, 1.77, 1.94},
+    {"a16w16_tile_64x64_bplain", 0.22, 0, 3.46, 0.01},
+    {"a16w16_skinny_m32_n32_bplain_lds", 0.04, 0.000485, 3.87, 0.01},
+    {"a16w16_skinny_m64_n32_bplain_lds", 0.137, 0.195, 1.53, 0.497},
+    {"a16w16_skinny_m64_bplain", 0.246, 0.267, 2.77, 0.01},
+    {"a16w16_skinny_m32_bplain", 0.17, 0.174, 2.14, 0.729},
+    {"a16w16_tile_256x256_persist", 1.17, 0, 0.5, 7.59},
+    {"a16w16_tile_128x256_persist", 0.694, 0, 0.5, 5.22},
+    {"a16w16_tile_128x256", 0.696, 0, 0.5, 6.38},
+    {"a16w16_tile_160x128", 0.583, 0, 1.22, 2.65},
+    {"a16w16_tile_256x128", 0.742, 0, 0.5, 5.81},
+    {"a16w16_tile_256x256", 1.2, 0, 0.5, 9.78},
+    {"a16w16_tile_128x128", 0.455, 0, 0.798, 3.26},
+    {"a16w16_tile_160x128_splitk", 0.583, 0, 5.53, 0.01},
+    {"a16w16_tile_96x128", 0.391, 0, 0.625, 2.44},
+    {"a16w16_tile_96x128_splitk", 0.395, 0, 5.91, 0.01},
+    {"a16w16_tile_64x128", 0.262, 0, 1.19, 2.45},
+    {"a16w16_tile_128x64_splitk", 0.354, 0, 4.22, 0.931},
+    {"a16w16_tile_128x64", 0.275, 0, 0.617, 2.96},
+    {"a16w16_tile_128x128_splitk", 0.49, 0, 5.79, 0.01},
+    {"a16w16_tile_64x128_splitk", 0.274, 0, 6.65, 0.01},
+    {"a16w16_tile_64x64_splitk", 0.236, 0, 5.82, 0.0154},
+    {"a16w16_skinny_m32", 0.113, 0.000332, 2.45, 0.125},
+    {"a16w16_skinny_m32_n32_alds", 0.0428, 0.0399, 3.64, 0.01},
+    {"a16w16_tile_64x64", 0.21, 0, 3.57, 0.01},
+    {"a16w16_skinny_m32_n32", 0.167, 0.189, 0.712, 0.581},
+    {"a16w16_skinny_m64_n32_alds", 0.113, 0.185, 1.04, 0.679},
+    {"a16w16_skinny_m64", 0.131, 0.195, 2.26, 0.911},
+};
+
+}  // namespace aiter_amd

@@ -41,6 +41,9 @@ struct Instance {
     bool persistent = false;   // grid of min(tiles, CUs) workgroups walking the tiles
     int rank = 0;              // among skinny forms of one shape the heuristic takes the highest
     bool stream_k = false;     // skinny stream-K form: one workgroup per CU, partial blocks summed in place
+    bool by_ref = true;        // may stand for a reference kernel of the same tile
+    bool listed = true;        // in the kernel table (unlisted instances come last and are run by name or dispatch)
+    const struct GemmCost* cost = nullptr;   // time model (gemm_cost.h); null: never the model's choice
 };
 
 template <int KA, int KB, int BM, int BN, bool AP, bool BP, bool OF>
@@ -193,6 +196,7 @@ struct RegBuilder {
     void part_rest();                  // gemm_reg_rest.hip
     void part_direct();                // gemm_reg_direct.hip
     void part_late();                  // gemm_reg_late.hip
+    void part_mid();                   // gemm_reg_mid.hip
 };
 
 constexpr Variant kPre{false, true, false}, kPlain{false, false, false}, kPre32{false, true, true};

@@ -17,7 +17,7 @@ from torch import Tensor
 
 from . import dtypes
 from ._lib import call
-from .config import A4W4_KEYS, DEFAULT_A4W4_CSV, get_cu_num, get_gfx, load_tuned
+from .config import A4W4_KEYS, DEFAULT_A4W4_CSV, get_cu_num, get_gfx, load_tuned, row_kernel, tuned_row
 from .gemm_common import get_padded_m
 
 logger = logging.getLogger("aiter_amd")
@@ -48,7 +48,7 @@ def get_GEMM_config(M: int, N: int, K: int):
         if cfg is not None:
             if AITER_LOG_TUNED_CONFIG:
                 logger.info(f"shape M:{M} N:{N} K:{K} tuned as padded_M {pm}: {cfg['kernelName']}")
-            return cfg
+            return tuned_row(cfg, M, pm, "AITER_CONFIG_GEMM_A4W4")
     logger.debug(f"shape M:{M} N:{N} K:{K} not tuned, using the heuristic")
     return None
 
@@ -104,6 +104,8 @@ def _gemm_a4w4_into(A: Tensor, B: Tensor, A_scale: Tensor, B_scale: Tensor, out:
             gemm_a4w4_blockscale(A.view(m, k // 2), B, A_scale, B_scale, out, splitK=split_k,
                                  kernelName=kernel_name)
             return
+        if kernel_name and _is_library_name(kernel_name):
+            kernel_name = row_kernel(cfg, m)
         gemm_a4w4_asm(A.view(m, k // 2), B, A_scale, B_scale, out, kernel_name, bias, alpha, beta,
                       bpreshuffle, log2_k_split=split_k)
     except RuntimeError as e:

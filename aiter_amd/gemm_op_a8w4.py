@@ -16,7 +16,7 @@ from torch import Tensor
 
 from . import dtypes
 from ._lib import call
-from .config import A4W4_KEYS, DEFAULT_A8W4_CSV, get_cu_num, get_gfx, load_tuned
+from .config import A4W4_KEYS, DEFAULT_A8W4_CSV, get_cu_num, get_gfx, load_tuned, row_kernel, tuned_row
 from .gemm_common import get_padded_m
 from .quant import per_1x32_mx_quant_hip, dynamic_mxfp8_quant
 from .shuffle import shuffle_weight
@@ -37,7 +37,7 @@ def get_GEMM_A8W4_config(M: int, N: int, K: int):
         pm = M if gl is None else get_padded_m(M, N, K, gl)
         cfg = table.get((gfx, cu_num, pm, N, K))
         if cfg is not None:
-            return cfg
+            return tuned_row(cfg, M, pm, "AITER_CONFIG_GEMM_A8W4")
     return None
 
 
@@ -51,7 +51,7 @@ def gemm_a8w4_mxfp8(A: Tensor, B: Tensor, ScaleA: Tensor, ScaleB: Tensor, dtype:
     if not kernelName and not a_preshuffle:
         cfg = get_GEMM_A8W4_config(M, N, A.shape[1])
         if cfg is not None:
-            kernelName = str(cfg["kernelName"])
+            kernelName = row_kernel(cfg, M)
     call("mxfp8_mxfp4_gemm_asm", A, B, ScaleA, ScaleB, out, kernelName if kernelName else None,
          int(bool(a_preshuffle)))
     return out

@@ -26,7 +26,7 @@ from torch import Tensor
 
 from . import dtypes
 from ._lib import call
-from .config import BF16_KEYS, DEFAULT_BF16_CSV, get_cu_num, get_gfx, load_tuned
+from .config import BF16_KEYS, DEFAULT_BF16_CSV, TunedRow, get_cu_num, get_gfx, load_tuned, row_kernel, tuned_row
 from .gemm_common import get_padded_m
 
 AITER_TUNE_GEMM = int(os.environ.get("AITER_TUNE_GEMM", "0"))
@@ -52,7 +52,7 @@ def get_GEMM_A16W16_config(M: int, N: int, K: int, bias: bool, dtype: str, otype
         pm = M if gl is None else get_padded_m(M, N, K, gl)
         cfg = table.get((gfx, cu, pm, N, K, bias, dtype, otype, scaleAB, bpreshuffle))
         if cfg is not None:
-            return cfg
+            return tuned_row(cfg, M, pm, "AITER_CONFIG_GEMM_BF16")
     return _default_config()
 
 
@@ -72,7 +72,7 @@ def _run(inp: Tensor, B: Tensor, bias: Tensor | None, otype: torch.dtype, bpresh
              int(config.get("solidx", -1)), split)
         return out
     if libtype == "aiter_amd" and int(config.get("solidx", -1)) >= 0:
-        name = str(config.get("kernelName", ""))
+        name = row_kernel(config, m) if isinstance(config, TunedRow) else str(config.get("kernelName", ""))
     elif libtype == "asm":
         name = str(config.get("kernelName", "") or "")
     else:

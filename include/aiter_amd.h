@@ -73,7 +73,9 @@ int getPaddedM(int M, int N, int K, int gl);
  * library's table; or a reference kernel name (ASM "_ZN5aiter..._<tM>x<tN>E",
  * CK "a4w4_blockscale_<block>x<tM>x<tN>x<tK>_..."), which runs the tile of
  * the same shape here when there is one and M > 32, else the heuristic
- * choice; "" or NULL = heuristic; any other name is an error.
+ * choice; "" or NULL = heuristic; "~<name>" (any GEMM entry) = that kernel
+ * unless the library's time model puts another clearly below it (a row tuned
+ * for other row counts); any other name is an error.
  * log2_k_split <= 0 lets the heuristic choose the split-K factor. */
 int gemm_a4w4_asm(aiter_tensor_t* A, aiter_tensor_t* B, aiter_tensor_t* A_scale,
                   aiter_tensor_t* B_scale, aiter_tensor_t* out, const char* kernelName,
