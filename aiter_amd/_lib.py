@@ -123,6 +123,8 @@ SIGNATURES = {
                                   ctypes.c_int, ctypes.c_int, _S], ctypes.c_int),
     "ck_moe_stage2": ([_T] * 7 + [ctypes.c_int, ctypes.c_char_p, _T, _T, ctypes.c_int, _T] + [ctypes.c_int] * 4
                       + [ctypes.c_char_p, ctypes.c_int, _S], ctypes.c_int),
+    "moe_stage1_stream": ([_T] * 7 + [ctypes.c_int, _T, _T, ctypes.c_int, _T, _T, ctypes.c_int, _S], ctypes.c_int),
+    "moe_stage2_reduce": ([_T] * 6 + [ctypes.c_int, _T, _T, ctypes.c_int, _T, _S], ctypes.c_int),
     "moe_sum": ([_T, _T, _S], ctypes.c_int),
     "mxfp4_gemm_asm": ([_T] * 6 + [ctypes.c_char_p, ctypes.c_int, _S], ctypes.c_int),
     "batched_gemm_bf16": ([_T] * 4 + [ctypes.c_int, _S], ctypes.c_int),

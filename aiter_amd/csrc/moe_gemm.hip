@@ -10,7 +10,9 @@
 #include "gemm_kernels.h"
 #include "mfma32.h"
 #include "gemm_flat.h"
+#include "moe_stage1_stream.h"
 #include "moe_stage2.h"
+#include "moe_stage2_reduce.h"
 
 namespace {
 
@@ -26,6 +28,8 @@ struct StageArgs {
     // q_w the sorted routing weights of the zero-row rule (optional)
     aiter_tensor_t* q_scale = nullptr;
     aiter_tensor_t* q_w = nullptr;
+    bool reduce = false;   // stage 2 that writes each token's sum over its slots
+    bool stream = false;   // stage 1 on the weight-streaming kernel (fused quant only)
 };
 
 template <int KA, int MOE>
@@ -197,6 +201,11 @@ void run_stage(const StageArgs& s, hipStream_t st) {
         tiles_n = (int)(model_dim / 256);
     }
     AA_CHECK(mq.out_stride % 4 == 0, "out rows must be 8-byte aligned");
+    if (s.reduce)
+        AA_CHECK(!a_fp8 && (K == 256 || K == 512) && s.out->ndim == 2 && mq.out_stride % 8 == 0 &&
+                     ((uintptr_t)s.out->ptr & 15) == 0 && token_num <= kS2ReduceTokens,
+                 "moe_stage2_reduce: at most ", kS2ReduceTokens,
+                 " tokens, MXFP4 rows of K = 256 or 512, 16-byte aligned rows of a 2-D out");
 
     GemmParams p{};
     p.A = static_cast<const uint8_t*>(s.a->ptr);
@@ -215,6 +224,12 @@ void run_stage(const StageArgs& s, hipStream_t st) {
     p.tiles_n = tiles_n;
     p.alpha = 1.0f;
 
+    if (s.reduce) {
+        if (token_num == 0) return;
+        launch_stage2_reduce(p, mq, device_cu_count(s.out->device_id), st);
+        AA_HIP(hipGetLastError());
+        return;
+    }
     // row blocks in use are at most ceil(entries / block_m) + (experts hit);
     // blocks past num_valid_ids[0] leave at once
     const int64_t entries = token_num * s.topk;
@@ -224,6 +239,12 @@ void run_stage(const StageArgs& s, hipStream_t st) {
     if (used == 0) return;
     p.tiles_m = (int)used;
     AA_CHECK((int64_t)tiles_n * used < ((int64_t)1 << 31), "grid too large");
+    if (s.stream) {
+        AA_CHECK(fq && !a_fp8, "moe_stage1_stream: MXFP4 activations and output");
+        launch_stage1_stream(p, mq, used_sort * (s.block_m / 32), entries, device_cu_count(s.out->device_id), st);
+        AA_HIP(hipGetLastError());
+        return;
+    }
     // stage-1 split-K while the tiles leave the CUs short of weight loads in
     // flight (decode and small batches; at least 2 K stages per split).  A
     // workgroup keeps one K stage of B ahead, so a CU with one tile streams
@@ -375,6 +396,34 @@ int ck_moe_stage1_fuse_quant(aiter_tensor_t* hidden_states, aiter_tensor_t* w1, 
         StageArgs s{hidden_states, w1, a1_scale, w1_scale, sorted_token_ids, sorted_expert_ids, num_valid_ids, out,
                     sorted_weights, topk, block_m, activation, 1, splitk, tile_from_name(kernelName, 1, block_m),
                     kernelName, out_scale, quant_weights};
+        run_stage(s, reinterpret_cast<hipStream_t>(stream));
+    });
+}
+
+int moe_stage1_stream(aiter_tensor_t* hidden_states, aiter_tensor_t* w1, aiter_tensor_t* sorted_token_ids,
+                      aiter_tensor_t* sorted_expert_ids, aiter_tensor_t* num_valid_ids, aiter_tensor_t* out,
+                      aiter_tensor_t* out_scale, int topk, aiter_tensor_t* w1_scale, aiter_tensor_t* a1_scale,
+                      int block_m, aiter_tensor_t* sorted_weights, aiter_tensor_t* quant_weights, int activation,
+                      aiter_stream_t stream) {
+    return safe_call([&] {
+        AA_CHECK(out_scale, "moe_stage1_stream: out_scale must be given");
+        DeviceGuard g(hidden_states ? hidden_states->device_id : -1);
+        StageArgs s{hidden_states, w1, a1_scale, w1_scale, sorted_token_ids, sorted_expert_ids, num_valid_ids, out,
+                    sorted_weights, topk, block_m, activation, 1, 1, block_m, nullptr, out_scale, quant_weights};
+        s.stream = true;
+        run_stage(s, reinterpret_cast<hipStream_t>(stream));
+    });
+}
+
+int moe_stage2_reduce(aiter_tensor_t* inter_states, aiter_tensor_t* w2, aiter_tensor_t* sorted_token_ids,
+                      aiter_tensor_t* sorted_expert_ids, aiter_tensor_t* num_valid_ids, aiter_tensor_t* out, int topk,
+                      aiter_tensor_t* w2_scale, aiter_tensor_t* a2_scale, int block_m,
+                      aiter_tensor_t* sorted_weights, aiter_stream_t stream) {
+    return safe_call([&] {
+        DeviceGuard g(inter_states ? inter_states->device_id : -1);
+        StageArgs s{inter_states, w2, a2_scale, w2_scale, sorted_token_ids, sorted_expert_ids, num_valid_ids, out,
+                    sorted_weights, topk, block_m, 0, 2, 1, std::min(block_m, 64), nullptr};
+        s.reduce = true;
         run_stage(s, reinterpret_cast<hipStream_t>(stream));
     });
 }

@@ -273,6 +273,19 @@ def ck_moe_stage1_fuse_quant(hidden_states, w1, sorted_token_ids, sorted_expert_
     return a2, a2_scale
 
 
+def moe_stage1_stream(hidden_states, w1, sorted_token_ids, sorted_expert_ids, num_valid_ids, token_num: int, topk: int,
+                      block_m: int, w1_scale, a1_scale, sorted_weights=None, quant_weights=None, activation: int = 0):
+    """ck_moe_stage1_fuse_quant on the kernel for few rows per expert (MXFP4
+    activations): same results up to the order of the f32 sums."""
+    inter_dim = w1.shape[1] // 2
+    a2 = torch.empty((token_num, topk, inter_dim // 2), dtype=dtypes.fp4x2, device=hidden_states.device)
+    a2_scale = _sorted_scale(sorted_token_ids, inter_dim, hidden_states.device)
+    call("moe_stage1_stream", _u8(hidden_states), _u8(w1), sorted_token_ids, sorted_expert_ids, num_valid_ids,
+         _u8(a2.view(-1, a2.shape[-1])), _u8(a2_scale), int(topk), _u8(w1_scale), _u8(a1_scale), int(block_m),
+         sorted_weights, quant_weights, int(activation))
+    return a2, a2_scale
+
+
 def ck_moe_stage2(inter_states, w1, w2, sorted_token_ids, sorted_expert_ids, num_valid_ids, out, topk: int,
                   kernelName: str | None = None, w2_scale=None, a2_scale=None, block_m: int | None = 32,
                   sorted_weights=None, quant_type: int = 0, activation: int = 0, splitk: int = 1,
@@ -287,6 +300,17 @@ def ck_moe_stage2(inter_states, w1, w2, sorted_token_ids, sorted_expert_ids, num
     call("ck_moe_stage2", a, None, _u8(w2), sorted_token_ids, sorted_expert_ids, num_valid_ids, out, int(topk),
          kernelName or "", _u8(w2_scale), _u8(a2_scale), int(block_m or 32), sorted_weights, int(quant_type),
          int(activation), int(splitk), int(bool(use_non_temporal_load)), dst_type, int(bool(is_shuffled)))
+
+
+def moe_stage2_reduce(inter_states, w2, sorted_token_ids, sorted_expert_ids, num_valid_ids, out, topk: int, w2_scale,
+                      a2_scale, block_m: int, sorted_weights=None) -> None:
+    """Stage 2 and the sum over the slots in one launch: out [token_num,
+    model_dim] bf16 = sum over the token's routed pairs of weight * (a2 row @
+    w2[expert]^T), summed in f32 (in any order) and rounded once; every row is
+    written.  a2 MXFP4 with inter_dim 256 or 512."""
+    a = _u8(inter_states.view(-1, inter_states.shape[-1]))
+    call("moe_stage2_reduce", a, _u8(w2), sorted_token_ids, sorted_expert_ids, num_valid_ids, out, int(topk),
+         _u8(w2_scale), _u8(a2_scale), int(block_m), sorted_weights)
 
 
 def moe_sum(input: torch.Tensor, output: torch.Tensor) -> None:
@@ -325,26 +349,31 @@ def fused_moe_2stages(hidden_states, w1, w2, topk, sorted_ids, sorted_weights, s
                       num_local_tokens=None, expert_mask=None, a1=None, a1_scale=None):
     """The per_1x32 two-stage flow of aiter/fused_moe.py:2892-3276: quant +
     sort of the tokens, stage 1, quant + sort of the stage-1 output, stage 2
-    accumulating into ``moe_out``.  ``a1`` / ``a1_scale``: the tokens already
+    accumulating into ``moe_out`` (or overwriting it, from REDUCE_MIN_ROWS routed
+    rows; an empty ``moe_out`` is allocated).  ``a1`` / ``a1_scale``: the tokens already
     quantised with their scales in sorted order (moe_sorting_mx_quant)."""
     token_num = hidden_states.shape[0]
     E, model_dim, inter_dim = get_inter_dim(w1.shape, w2.shape)
     # per-pair rows miss the pairs routed to masked experts or past
     # num_local_tokens, so those cases accumulate (as in the reference)
-    reduce = expert_mask is None and num_local_tokens is None and _use_reduce(token_num, topk)
+    whole = expert_mask is None and num_local_tokens is None
+    reduce = whole and _use_reduce(token_num, topk)
+    # rows handed in for accumulation are added to; rows of the reduced forms are overwritten
+    summed = (whole and _sum_in_stage2(token_num, topk, model_dim, inter_dim, q_dtype_a) and
+              (moe_out.numel() == 0 or (reduce and moe_out.is_contiguous() and moe_out.data_ptr() % 16 == 0)))
     if moe_out.numel() == 0:
         moe_out = torch.empty((token_num, model_dim), dtype=dtypes.bf16, device=hidden_states.device)
     if a1 is None:
         a1, a1_scale = fused_dynamic_mx_quant_moe_sort(hidden_states, sorted_ids, num_valid_ids, token_num, topk,
                                                        block_size_M, q_dtype_a, num_rows=num_local_tokens,
                                                        sorted_weights=sorted_weights)
-    if q_dtype_a == dtypes.fp4x2 and inter_dim % 256 == 0 and expert_mask is None and num_local_tokens is None:
+    if q_dtype_a == dtypes.fp4x2 and inter_dim % 256 == 0 and whole:
         # fuse_quant "fp4": stage 1 writes its output already quantised (one
         # launch and one pass over the stage-1 output less)
-        a2q, a2_scale = ck_moe_stage1_fuse_quant(a1, w1, sorted_ids, sorted_expert_ids, num_valid_ids, token_num,
-                                                 topk, block_size_M, w1_scale, a1_scale,
-                                                 sorted_weights if doweight_stage1 else None, sorted_weights,
-                                                 int(activation))
+        stage1 = moe_stage1_stream if _stream_stage1(token_num, topk, E) else ck_moe_stage1_fuse_quant
+        a2q, a2_scale = stage1(a1, w1, sorted_ids, sorted_expert_ids, num_valid_ids, token_num, topk, block_size_M,
+                               w1_scale, a1_scale, sorted_weights if doweight_stage1 else None, sorted_weights,
+                               int(activation))
     else:
         a2 = torch.empty((token_num, topk, inter_dim), dtype=dtypes.bf16, device=hidden_states.device)
         ck_moe_stage1(a1, w1, w2, sorted_ids, sorted_expert_ids, num_valid_ids, a2, topk, "", w1_scale, a1_scale,
@@ -353,7 +382,10 @@ def fused_moe_2stages(hidden_states, w1, w2, topk, sorted_ids, sorted_weights, s
         a2q, a2_scale = fused_dynamic_mx_quant_moe_sort(a2.view(-1, inter_dim), sorted_ids, num_valid_ids,
                                                         token_num, topk, block_size_M, q_dtype_a,
                                                         sorted_weights=sorted_weights)
-    if reduce:
+    if summed:
+        moe_stage2_reduce(a2q, w2, sorted_ids, sorted_expert_ids, num_valid_ids, moe_out, topk, w2_scale, a2_scale,
+                          block_size_M, None if doweight_stage1 else sorted_weights)
+    elif reduce:
         # one row per routed pair, then a fixed-order sum over the slots: device-
         # wide atomics cost one memory-side operation per 4 bytes, which
         # dominates once there are more than a few hundred routed rows
@@ -373,6 +405,41 @@ REDUCE_MIN_ROWS = 128
 def _use_reduce(token_num: int, topk: int) -> bool:
     """Per-pair rows + moe_sum instead of atomics: from REDUCE_MIN_ROWS routed rows."""
     return token_num * topk >= REDUCE_MIN_ROWS
+
+
+STREAM_ROWS_PER_EXPERT = 3
+
+
+def _stream_stage1(token_num: int, topk: int, experts: int) -> bool:
+    """Stage 1 on the weight-streaming kernel: up to 3 routed rows per expert.
+
+    us per launch, flat kernel / streaming kernel (experts, topk, model_dim,
+    inter_dim; tokens): 257, 9, 7168, 256: 10.9 / 9.5 at 1, 31.6 / 22.3 at 8,
+    85 / 67 at 64 (2.2 rows per expert), 93 / 104 at 100 (3.5); 256, 8, 3072,
+    256: 22.3 / 19.0 at 16, 49 / 34 at 100 (3.1), 45.6 / 47.6 at 128 (4); 128,
+    8, 4096, 512: 19.0 / 14.1 at 4, 53 / 41 at 48 (3), 58 / 65 at 100 (6.3).
+    Past that an item's 16-row halves both hold rows and its weights are read
+    by two waves, where the flat kernel shares them through LDS."""
+    return token_num * topk <= STREAM_ROWS_PER_EXPERT * experts
+
+
+SUM_IN_STAGE2_TOKENS = 128
+
+
+def _sum_in_stage2(token_num: int, topk: int, model_dim: int, inter_dim: int, q_dtype_a) -> bool:
+    """Stage 2 with the sum over the slots in the same launch: MXFP4 rows, K of
+    256 or 512, up to 128 tokens (their f32 sums fit the LDS).
+
+    us of the two steps it replaces (rows + sum; atomics below 128 rows) / it:
+    257 experts, topk 9, 7168 x 256: 6.7 / 5.4 at 1 token, 22.5 / 14.4 at 8,
+    54 / 36 at 64, 57 / 45 at 100; 512, 10, 4096 x 256: 24.4 / 18.1 at 16, 62 /
+    42 at 100; 128, 8, 4096 x 512: 12.6 / 10.0 at 4, 35 / 26 at 48; 256, 8,
+    3072 x 256: 25.2 / 21.4 at 48, 27.3 / 26.6 at 128.  Narrower outputs take
+    16-column workgroups, where a few rows' atomics are the shorter way: 4096 x
+    256 7.6 / 8.7 at 40 rows, 3072 x 256 6.8 / 7.7 at 32, 1536 x 256 9.0 / 7.5
+    at 128."""
+    return (q_dtype_a == dtypes.fp4x2 and inter_dim in (256, 512) and 0 < token_num <= SUM_IN_STAGE2_TOKENS and
+            (token_num * topk >= 64 or model_dim >= 6144))
 
 
 def fused_moe(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask=None, activation=ActivationType.Silu,
@@ -409,7 +476,9 @@ def fused_moe(hidden_states, w1, w2, topk_weight, topk_ids, expert_mask=None, ac
     global_E = expert_mask.numel() if expert_mask is not None else E
     bm = block_size_M if block_size_M and block_size_M > 0 else get_block_size_M(token_num, topk, global_E,
                                                                                  inter_dim)
-    accumulate = not (expert_mask is None and num_local_tokens is None and _use_reduce(token_num, topk))
+    accumulate = not (expert_mask is None and num_local_tokens is None and
+                      (_use_reduce(token_num, topk) or
+                       _sum_in_stage2(token_num, topk, model_dim, inter_dim, dtypes.fp4x2)))
     a1 = a1_scale = None
     if can_sort_quant(hidden_states, topk_ids, expert_mask, num_local_tokens, moe_sorting_dispatch_policy):
         # decode: the sort and the token quant in one launch

@@ -570,7 +570,10 @@ def _moe_stage_times(aiter_amd, x, w1, w2, w1s, w2s, tw, ti, E, topk, dim, inter
 
     m = x.shape[0]
     bm = FM.get_block_size_M(m, topk, E, inter)
-    reduce = FM._use_reduce(m, topk)
+    # the forms fused_moe takes at this size
+    summed = FM._sum_in_stage2(m, topk, dim, inter, dtypes.fp4x2)
+    reduce = FM._use_reduce(m, topk) or summed
+    stage1 = FM.moe_stage1_stream if FM._stream_stage1(m, topk, E) else FM.ck_moe_stage1_fuse_quant
     qt = int(aiter_amd.QuantType.per_1x32)
     sort = lambda: FM.moe_sorting(ti, tw, E, dim, torch.bfloat16, bm, None, None, 0, accumulate=not reduce)
     sids, sw, seids, nv, moe_buf = sort()
@@ -578,8 +581,7 @@ def _moe_stage_times(aiter_amd, x, w1, w2, w1s, w2s, tw, ti, E, topk, dim, inter
     a1, a1s = q1()
     # stage 1 with its output quantised in the same launch (the flow fused_moe
     # takes here; the reference's fuse_quant "fp4" stage 1)
-    s1 = lambda: FM.ck_moe_stage1_fuse_quant(a1, w1, sids, seids, nv, m, topk, bm, w1s, a1s, None, sw,
-                                             int(FM.ActivationType.Silu))
+    s1 = lambda: stage1(a1, w1, sids, seids, nv, m, topk, bm, w1s, a1s, None, sw, int(FM.ActivationType.Silu))
     a2q, a2s = s1()
     if FM.can_sort_quant(x, ti):
         # decode: fused_moe sorts and quantises the tokens in one launch
@@ -589,7 +591,12 @@ def _moe_stage_times(aiter_amd, x, w1, w2, w1s, w2s, tw, ti, E, topk, dim, inter
     else:
         res = {"sort_us": time_graph(sort, 10, 2), "quant1_us": time_graph(q1, 10, 2), "sort_quant_fused": False}
     res.update({"stage1_us": time_graph(s1, 10, 2), "quant2_us": 0.0})
-    if reduce:
+    if summed:
+        moe_out = torch.empty((m, dim), dtype=torch.bfloat16, device=x.device)
+        res["stage2_us"] = time_graph(
+            lambda: FM.moe_stage2_reduce(a2q, w2, sids, seids, nv, moe_out, topk, w2s, a2s, bm, sw), 10, 2)
+        res["moe_sum_us"] = 0.0
+    elif reduce:
         per_pair = torch.empty((m, topk, dim), dtype=torch.bfloat16, device=x.device)
         s2 = lambda: FM.ck_moe_stage2(a2q, w1, w2, sids, seids, nv, per_pair, topk, "", w2s, a2s, bm, sw, qt)
         s2()

@@ -326,6 +326,24 @@ int ck_moe_stage1_fuse_quant(aiter_tensor_t* hidden_states, aiter_tensor_t* w1, 
                              aiter_tensor_t* out_scale, int topk, const char* kernelName, aiter_tensor_t* w1_scale,
                              aiter_tensor_t* a1_scale, int block_m, aiter_tensor_t* sorted_weights,
                              aiter_tensor_t* quant_weights, int activation, int splitk, aiter_stream_t stream);
+/* ck_moe_stage1_fuse_quant on a kernel for few rows per expert (MXFP4
+ * activations; sums in another order, so a code next to a rounding boundary
+ * may differ by one step). */
+int moe_stage1_stream(aiter_tensor_t* hidden_states, aiter_tensor_t* w1, aiter_tensor_t* sorted_token_ids,
+                      aiter_tensor_t* sorted_expert_ids, aiter_tensor_t* num_valid_ids, aiter_tensor_t* out,
+                      aiter_tensor_t* out_scale, int topk, aiter_tensor_t* w1_scale, aiter_tensor_t* a1_scale,
+                      int block_m, aiter_tensor_t* sorted_weights, aiter_tensor_t* quant_weights, int activation,
+                      aiter_stream_t stream);
+/* Stage 2 that writes each token's sum over its slots (no reference
+ * counterpart as one entry: stage 2 in its reduce mode followed by moe_sum,
+ * aiter/ops/moe_op.py:87-98).  inter_states fp4x2 [token_num * topk, inter / 2]
+ * with inter 256 or 512, out bf16 [token_num, model_dim] (every row written,
+ * zeros for a token without routed rows), f32 sums; the rest as
+ * ck_moe_stage2. */
+int moe_stage2_reduce(aiter_tensor_t* inter_states, aiter_tensor_t* w2, aiter_tensor_t* sorted_token_ids,
+                      aiter_tensor_t* sorted_expert_ids, aiter_tensor_t* num_valid_ids, aiter_tensor_t* out, int topk,
+                      aiter_tensor_t* w2_scale, aiter_tensor_t* a2_scale, int block_m,
+                      aiter_tensor_t* sorted_weights, aiter_stream_t stream);
 int ck_moe_stage2(aiter_tensor_t* inter_states, aiter_tensor_t* w1, aiter_tensor_t* w2,
                   aiter_tensor_t* sorted_token_ids, aiter_tensor_t* sorted_expert_ids, aiter_tensor_t* num_valid_ids,
                   aiter_tensor_t* out, int topk, const char* kernelName, aiter_tensor_t* w2_scale,

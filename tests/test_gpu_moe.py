@@ -24,6 +24,8 @@
 Weights are random fp4 bytes with scale bytes near 2^-6 (no CPU quant of
 large weight tensors); activations are randn bf16.
 """
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -514,3 +516,84 @@ def test_fused_moe_model_shapes(cuda, m, model):
     # by one fp4 step, so with inter_dim 2048 more outputs leave 1e-2 while
     # logits_diff stays far below its bound (1.1e-5 for GLM-5 at one token)
     _accept(out.float().cpu().numpy()[toks], ref, min_close=0.9 if inter <= 256 else 0.85)
+
+
+def _mxfp4_values(codes, scales, s, m, topk, inter):
+    """[m * topk, inter] f32 of e2m1 rows and their sorted scale bytes, and the scale of each element"""
+    plain = np.zeros((m * topk, inter // 32), np.uint8)
+    sc = O.unshuffle_scale(scales, len(scales), inter // 32)
+    for pos, v in enumerate(s):
+        t, k = int(v) & 0xffffff, int(v) >> 24 & 0xff
+        if t < m and pos < len(sc):
+            plain[t * topk + k] = sc[pos]
+    return O.dequant_mxfp4(codes, plain), np.repeat(np.exp2(plain.astype(np.float32) - 127.0), 32, axis=1)
+
+
+@pytest.mark.parametrize("m,e,topk,dim,inter,bs,act,doweight",
+                         [(1, 257, 9, 7168, 256, 32, 0, False), (2, 40, 8, 512, 512, 32, 1, True),
+                          (3, 40, 6, 768, 256, 64, 0, False), (17, 16, 3, 2304, 256, 32, 0, False),
+                          (64, 300, 9, 1280, 512, 32, 0, True), (48, 8, 4, 256, 256, 128, 1, False)])
+def test_stage1_stream(cuda, m, e, topk, dim, inter, bs, act, doweight):
+    """moe_stage1_stream against the flat kernel's fused quant: one launch of
+    one row half and of two, 1 to 8 waves over K, windows left over, experts
+    with more rows than a unit.  The f32 sums run in another order, so a value
+    on a rounding boundary may take the next e2m1 code (at most 2 scales away;
+    the larger of the two scales) and nothing else; that is rare (< 0.5 %)."""
+    import aiter_amd
+
+    FM = sys.modules["aiter_amd.fused_moe"]
+    announce(f"moe_stage1_stream m={m} e={e} topk={topk} dim={dim} inter={inter} bs={bs} act={act} dw={doweight}")
+    rng, ids, w, (s, sw, se, nv, _) = _stage_setup(m, e, topk, dim, inter, bs, 8100 + m, cuda, False)
+    sw[rng.integers(0, max(1, m * topk // 4))] = 0.0
+    aq, a_s = O.quant_mxfp4(to_bf16_f32(rng.standard_normal((m, dim)).astype(np.float32)), O.ROUND_UP,
+                            amax_floor=1e-10)
+    n = int(nv[0].item())
+    a_sorted = _dev(MO.sort_scale_ref(a_s, s.cpu().numpy(), n, m, 1), cuda)
+    w1d, w1sd = _w_dev(*_weights(e, 2 * inter, dim, rng), cuda)
+    args = (_dev(aq, cuda), w1d, s, se, nv, m, topk, bs, w1sd, a_sorted, sw if doweight else None, sw, act)
+    out = []
+    for fn in (FM.ck_moe_stage1_fuse_quant, FM.moe_stage1_stream):
+        q, sc = fn(*args)
+        torch.cuda.synchronize()
+        out.append(_mxfp4_values(q.view(torch.uint8).cpu().numpy().reshape(m * topk, -1),
+                                 sc.view(torch.uint8).cpu().numpy()[:(n + 31) // 32 * 32], s.cpu().numpy(), m, topk,
+                                 inter))
+    (ref, ref_scale), (got, got_scale) = out
+    step = 2.0 * np.maximum(ref_scale, got_scale)
+    assert np.all(np.abs(got - ref) <= step)
+    assert np.mean(got != ref) < 0.005
+
+
+@pytest.mark.parametrize("m", [1, 33, 64, 65, 128])
+@pytest.mark.parametrize("dim,inter", [(512, 256), (512, 512), (6144, 256), (6400, 512)])
+def test_stage2_reduce(cuda, m, dim, inter):
+    """moe_stage2_reduce against the oracle: 16- and 32-column workgroups, one
+    and two K windows, the smallest and largest token counts of each form;
+    tokens that route two slots to one expert, zero routing weights and a
+    token none of whose pairs exist.  Each output is one bf16 rounding of f32
+    sums (rtol = atol = 1e-2, as stage 2 with topk = 1)."""
+    FM = sys.modules["aiter_amd.fused_moe"]
+    announce(f"moe_stage2_reduce m={m} dim={dim} inter={inter}")
+    e, topk, bs = 12, 3, 32 if m < 65 else 64
+    rng = np.random.default_rng(8300 + m + dim + inter)
+    ids, w = _routing(m, e, topk, rng)
+    ids[rng.random(m) < 0.3, 1] = ids[0, 0]
+    ids[m // 2, 2] = ids[m // 2, 0]
+    w[rng.random(w.shape) < 0.1] = 0.0
+    s, sw, se, nv, _ = _sort_dev(ids, w, e, bs, cuda)
+    gone = m // 3 if m > 1 else None
+    if gone is not None:   # as if the sort had dropped them: the entry that names no token
+        s[(s & 0xffffff) == gone] = topk << 24 | m
+        w[gone] = 0.0
+    h = to_bf16_f32(rng.standard_normal((m * topk, inter)).astype(np.float32))
+    aq, a_s = O.quant_mxfp4(h, O.ROUND_UP, amax_floor=1e-10)
+    a_sorted = _dev(MO.sort_scale_ref(a_s, s.cpu().numpy(), int(nv[0].item()), m, topk), cuda)
+    w2q, w2s = _weights(e, dim, inter, rng)
+    w2d, w2sd = _w_dev(w2q, w2s, cuda)
+    out = torch.full((m, dim), float("nan"), dtype=torch.bfloat16, device=cuda)
+    FM.moe_stage2_reduce(_dev(aq, cuda), w2d, s, se, nv, out, topk, w2sd, a_sorted, bs, sw)
+    torch.cuda.synchronize()
+    ref = MO.moe_stage2_ref(O.dequant_mxfp4(aq, a_s).reshape(m, topk, inter), MO.dequant_experts(w2q, w2s), ids, w,
+                            True)
+    ok, msg = allclose_report(out.float().cpu().numpy(), O.bf16_bits_to_f32(O.f32_to_bf16_bits(ref)))
+    assert ok, msg
