@@ -1,8 +1,9 @@
-"""Build libaiter_amd.so (gfx950) in-tree with hipcc.
+"""Build libaiter_amd.so (gfx950) in-tree with hipcc, and _native.so, its caller
+for the Python package, with the host compiler against the installed torch.
 
 Usage: python -m aiter_amd.csrc.build   (or build() from Python)
-The library lands next to the package (aiter_amd/libaiter_amd.so) so it
-travels with the source tree.
+Both land next to the package (aiter_amd/libaiter_amd.so, aiter_amd/_native.so)
+so they travel with the source tree.
 """
 from __future__ import annotations
 
@@ -10,6 +11,7 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -18,6 +20,7 @@ ROOT = os.path.dirname(PKG)
 SOURCES = ["gemm.hip", "gemm_reg_mx.hip", "gemm_reg_bf16.hip", "gemm_reg_bf16_f32.hip", "gemm_reg_split.hip",
            "gemm_reg_rest.hip", "gemm_reg_direct.hip", "gemm_reg_late.hip", "gemm_reg_mid.hip", "quant.hip", "fused_quant.hip", "moe_sorting.hip", "moe_gemm.hip", "calib.hip"]
 LIB = os.path.join(PKG, "libaiter_amd.so")
+NATIVE = os.path.join(PKG, "_native.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 FLAGS = [
@@ -63,10 +66,41 @@ def _compile(src: str, out_dir: str, extra=()) -> tuple:
     return obj, vgpr_spills(r.stderr)
 
 
+def _compile_binding(out_dir: str) -> str:
+    import torch
+
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    obj = os.path.join(out_dir, "binding.o")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", inc, "-isystem",
+           os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem",
+           os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), "-isystem",
+           sysconfig.get_paths()["include"], "-I" + os.path.join(ROOT, "include"), "-c",
+           os.path.join(HERE, "binding.cpp"), "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"binding.cpp does not compile:\n{r.stderr[-6000:]}")
+    return obj
+
+
+def _link_binding(obj: str) -> None:
+    import torch
+
+    tmp = NATIVE + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-fPIC", "-o", tmp, obj, "-L" + PKG, "-l:libaiter_amd.so",
+           "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"_native.so does not link:\n{r.stderr[-4000:]}")
+    os.replace(tmp, NATIVE)
+
+
 def build(verbose: bool = True) -> str:
     out_dir = os.path.join(PKG, "_build")
     os.makedirs(out_dir, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
+    with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as ex:
+        binding = ex.submit(_compile_binding, out_dir)
         res = list(ex.map(lambda s: _compile(s, out_dir), SOURCES))
     objs = [o for o, _ in res]
     spills = {k: v for _, sp in res for k, v in sp.items()}
@@ -79,6 +113,7 @@ def build(verbose: bool = True) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
     os.replace(tmp, LIB)
+    _link_binding(binding.result())
     if verbose:
         print(f"built {LIB}")
         if spills:

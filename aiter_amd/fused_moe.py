@@ -52,10 +52,18 @@ class ActivationType(enum.IntEnum):
 BLOCK_SIZE_M = 32
 
 
+# element types that the library's data and scale arguments take as they are
+# (a view costs about 1 us of host time, a decode call has 14 such arguments)
+_DATA_DTYPES = (dtypes.fp4x2, torch.uint8)
+_SCALE_DTYPES = (dtypes.fp8_e8m0, torch.uint8)
+
+
 def _u8(t: torch.Tensor | None) -> torch.Tensor | None:
-    if t is None or t.dtype == torch.uint8:
-        return t
-    return t.view(torch.uint8)
+    return t if t is None or t.dtype in _DATA_DTYPES else t.view(torch.uint8)
+
+
+def _u8_scale(t: torch.Tensor | None) -> torch.Tensor | None:
+    return t if t is None or t.dtype in _SCALE_DTYPES else t.view(torch.uint8)
 
 
 # ------------------------------------------------------------------ sorting
@@ -112,7 +120,7 @@ def moe_sorting_mx_quant_fwd(topk_ids, topk_weights, hidden_states, sorted_token
     launch (decode-sized routing; the fusion of
     aiter/ops/flydsl/kernels/moe_fused_route_quant_scatter.py)."""
     call("moe_sorting_mx_quant", topk_ids, topk_weights, hidden_states, sorted_token_ids, sorted_weights,
-         sorted_expert_ids, num_valid_ids, moe_buf, _u8(a_out), _u8(a_scale), int(num_experts), int(unit_size))
+         sorted_expert_ids, num_valid_ids, moe_buf, _u8(a_out), _u8_scale(a_scale), int(num_experts), int(unit_size))
 
 
 def can_sort_quant(hidden_states, topk_ids, expert_mask=None, num_local_tokens=None, dispatch_policy=0) -> bool:
@@ -169,13 +177,14 @@ def _sorted_scale(sorted_ids: torch.Tensor, cols: int, device) -> torch.Tensor:
 def fused_dynamic_mx_quant_moe_sort_hip(out, scales, input, sorted_ids, num_valid_ids, token_num: int,
                                         block_m: int, group_size: int = 32, sorted_weights=None) -> None:
     """C entry (aiter/ops/quant.py:895-911)."""
-    call("fused_dynamic_mx_quant_moe_sort_hip", _u8(out) if out.dtype != dtypes.fp8 else out, _u8(scales), input,
-         sorted_ids, num_valid_ids, int(token_num), int(block_m), int(group_size), sorted_weights)
+    call("fused_dynamic_mx_quant_moe_sort_hip", _u8(out) if out.dtype != dtypes.fp8 else out, _u8_scale(scales),
+         input, sorted_ids, num_valid_ids, int(token_num), int(block_m), int(group_size), sorted_weights)
 
 
 def mxfp4_moe_sort_hip(out_scale, scale, sorted_ids, num_valid_ids, token_num: int, cols: int) -> None:
     """C entry (aiter/ops/quant.py:861-871): per-row e8m0 bytes -> sorted shuffled layout."""
-    call("mxfp4_moe_sort_hip", _u8(out_scale), _u8(scale), sorted_ids, num_valid_ids, int(token_num), int(cols))
+    call("mxfp4_moe_sort_hip", _u8_scale(out_scale), _u8_scale(scale), sorted_ids, num_valid_ids, int(token_num),
+         int(cols))
 
 
 def mxfp4_moe_sort_fwd(scale, sorted_ids, num_valid_ids, token_num: int, cols: int):
@@ -247,8 +256,8 @@ def ck_moe_stage1(hidden_states, w1, w2, sorted_token_ids, sorted_expert_ids, nu
     GPU, as in decode)."""
     a = hidden_states if hidden_states.dtype == dtypes.fp8 else _u8(hidden_states)
     call("ck_moe_stage1", a, _u8(w1), None, sorted_token_ids, sorted_expert_ids, num_valid_ids,
-         out.view(-1, out.shape[-1]), int(topk), kernelName or "", _u8(w1_scale), _u8(a1_scale), int(block_m or 32),
-         sorted_weights, int(quant_type), int(activation), int(1 if splitk is None else splitk),
+         out.view(-1, out.shape[-1]), int(topk), kernelName or "", _u8_scale(w1_scale), _u8_scale(a1_scale),
+         int(block_m or 32), sorted_weights, int(quant_type), int(activation), int(1 if splitk is None else splitk),
          int(bool(use_non_temporal_load)),
          dst_type, int(bool(is_shuffled)))
 
@@ -268,8 +277,8 @@ def ck_moe_stage1_fuse_quant(hidden_states, w1, sorted_token_ids, sorted_expert_
     a2_scale = _sorted_scale(sorted_token_ids, inter_dim, hidden_states.device)
     a = hidden_states if hidden_states.dtype == dtypes.fp8 else _u8(hidden_states)
     call("ck_moe_stage1_fuse_quant", a, _u8(w1), sorted_token_ids, sorted_expert_ids, num_valid_ids,
-         _u8(a2.view(-1, a2.shape[-1])), _u8(a2_scale), int(topk), kernelName or "", _u8(w1_scale), _u8(a1_scale),
-         int(block_m), sorted_weights, quant_weights, int(activation), int(splitk))
+         _u8(a2.view(-1, a2.shape[-1])), _u8_scale(a2_scale), int(topk), kernelName or "", _u8_scale(w1_scale),
+         _u8_scale(a1_scale), int(block_m), sorted_weights, quant_weights, int(activation), int(splitk))
     return a2, a2_scale
 
 
@@ -281,7 +290,7 @@ def moe_stage1_stream(hidden_states, w1, sorted_token_ids, sorted_expert_ids, nu
     a2 = torch.empty((token_num, topk, inter_dim // 2), dtype=dtypes.fp4x2, device=hidden_states.device)
     a2_scale = _sorted_scale(sorted_token_ids, inter_dim, hidden_states.device)
     call("moe_stage1_stream", _u8(hidden_states), _u8(w1), sorted_token_ids, sorted_expert_ids, num_valid_ids,
-         _u8(a2.view(-1, a2.shape[-1])), _u8(a2_scale), int(topk), _u8(w1_scale), _u8(a1_scale), int(block_m),
+         a2, a2_scale, int(topk), _u8_scale(w1_scale), _u8_scale(a1_scale), int(block_m),
          sorted_weights, quant_weights, int(activation))
     return a2, a2_scale
 
@@ -298,8 +307,9 @@ def ck_moe_stage2(inter_states, w1, w2, sorted_token_ids, sorted_expert_ids, num
     a = inter_states.view(-1, inter_states.shape[-1])
     a = a if a.dtype == dtypes.fp8 else _u8(a)
     call("ck_moe_stage2", a, None, _u8(w2), sorted_token_ids, sorted_expert_ids, num_valid_ids, out, int(topk),
-         kernelName or "", _u8(w2_scale), _u8(a2_scale), int(block_m or 32), sorted_weights, int(quant_type),
-         int(activation), int(splitk), int(bool(use_non_temporal_load)), dst_type, int(bool(is_shuffled)))
+         kernelName or "", _u8_scale(w2_scale), _u8_scale(a2_scale), int(block_m or 32), sorted_weights,
+         int(quant_type), int(activation), int(splitk), int(bool(use_non_temporal_load)), dst_type,
+         int(bool(is_shuffled)))
 
 
 def moe_stage2_reduce(inter_states, w2, sorted_token_ids, sorted_expert_ids, num_valid_ids, out, topk: int, w2_scale,
@@ -310,7 +320,7 @@ def moe_stage2_reduce(inter_states, w2, sorted_token_ids, sorted_expert_ids, num
     written.  a2 MXFP4 with inter_dim 256 or 512."""
     a = _u8(inter_states.view(-1, inter_states.shape[-1]))
     call("moe_stage2_reduce", a, _u8(w2), sorted_token_ids, sorted_expert_ids, num_valid_ids, out, int(topk),
-         _u8(w2_scale), _u8(a2_scale), int(block_m), sorted_weights)
+         _u8_scale(w2_scale), _u8_scale(a2_scale), int(block_m), sorted_weights)
 
 
 def moe_sum(input: torch.Tensor, output: torch.Tensor) -> None:

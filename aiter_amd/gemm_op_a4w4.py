@@ -16,7 +16,7 @@ import torch
 from torch import Tensor
 
 from . import dtypes
-from ._lib import call
+from ._lib import call, kernel_names
 from .config import A4W4_KEYS, DEFAULT_A4W4_CSV, get_cu_num, get_gfx, load_tuned, row_kernel, tuned_row
 from .gemm_common import get_padded_m
 
@@ -77,7 +77,8 @@ def gemm_a4w4(A: Tensor, B: Tensor, A_scale: Tensor, B_scale: Tensor, bias: Tens
     n = B.shape[0]
     out = torch.empty(((m + 31) // 32 * 32, n), dtype=dtype, device=A.device)
     _gemm_a4w4_into(A, B, A_scale, B_scale, out, bias, alpha, beta, bpreshuffle)
-    return out[:m].view(*A.shape[:-1], n)
+    rows = out if out.shape[0] == m else out[:m]
+    return rows if A.dim() == 2 else rows.view(*A.shape[:-1], n)
 
 
 def _gemm_a4w4_into(A: Tensor, B: Tensor, A_scale: Tensor, B_scale: Tensor, out: Tensor, bias: Tensor | None,
@@ -87,6 +88,7 @@ def _gemm_a4w4_into(A: Tensor, B: Tensor, A_scale: Tensor, B_scale: Tensor, out:
     m = A.numel() // A.shape[-1]
     n = B.shape[0]
     k = A.shape[-1] * 2
+    rows = A if A.dim() == 2 else A.view(m, k // 2)
     cfg = get_GEMM_config(m, n, k)
     split_k = 0
     kernel_name = ""
@@ -101,18 +103,18 @@ def _gemm_a4w4_into(A: Tensor, B: Tensor, A_scale: Tensor, B_scale: Tensor, out:
         if kernel_name and "_ZN" not in kernel_name and not _is_library_name(kernel_name):
             # a CK instance row: the reference sends every non-ASM name to the
             # CK entry, which takes no bias/alpha/beta (aiter/ops/gemm_op_a4w4.py:207-221)
-            gemm_a4w4_blockscale(A.view(m, k // 2), B, A_scale, B_scale, out, splitK=split_k,
+            gemm_a4w4_blockscale(rows, B, A_scale, B_scale, out, splitK=split_k,
                                  kernelName=kernel_name)
             return
         if kernel_name and _is_library_name(kernel_name):
             kernel_name = row_kernel(cfg, m)
-        gemm_a4w4_asm(A.view(m, k // 2), B, A_scale, B_scale, out, kernel_name, bias, alpha, beta,
+        gemm_a4w4_asm(rows, B, A_scale, B_scale, out, kernel_name, bias, alpha, beta,
                       bpreshuffle, log2_k_split=split_k)
     except RuntimeError as e:
         if not kernel_name or "unknown kernel name" not in str(e):
             raise
         _warn_unresolved(kernel_name, m, n, k)
-        gemm_a4w4_asm(A.view(m, k // 2), B, A_scale, B_scale, out, "", bias, alpha, beta, bpreshuffle,
+        gemm_a4w4_asm(rows, B, A_scale, B_scale, out, "", bias, alpha, beta, bpreshuffle,
                       log2_k_split=0)
 
 
@@ -129,8 +131,6 @@ def _warn_unresolved(name: str, m: int, n: int, k: int) -> None:
 
 
 def _is_library_name(name: str) -> bool:
-    from ._lib import kernel_names
-
     return name in kernel_names()
 
 
