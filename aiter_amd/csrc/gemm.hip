@@ -82,11 +82,10 @@ bool variant_ok(const Instance& in, Family f, const Variant& v) {
 }
 
 // Split-K factor for a skinny launch: split only when the 16-column blocks
-// cannot cover the CUs, keeping at least `per_split` k-steps (32: 8 per wave)
-// per split.
-int skinny_splits(int n_blocks, int k_steps, int cus, int per_split = 32) {
+// cannot cover the CUs, keeping at least 32 k-steps (8 per wave) per split.
+int skinny_splits(int n_blocks, int k_steps, int cus) {
     int s = 1;
-    while (n_blocks * s < cus && k_steps / (s * 2) >= per_split) s *= 2;
+    while (n_blocks * s < cus && k_steps / (s * 2) >= 32) s *= 2;
     return s;
 }
 
@@ -158,11 +157,17 @@ int tile_split_count(const Instance& in, int M, int N, int K, int cus, int want)
 // traffic is the larger part there; up to 16 rows only while they fit one
 // round, at N = 14336 two rounds of them measured 25.0 us against 21.2 in
 // bf16), else 16-column ones, unless only the 32-column form has its operands
-// copied through LDS (MXFP8: 6.3 against 8.8 us at 24 x 1088 x 7168).  K is
-// split only without an LDS form and from K = 16384 (MX) or 8192 (bf16) on: the
-// fill and finish launches cost 3 us (bf16 24 x 3072 x 6144 13.4 unsplit, 24.9
-// split; 1 x 256 x 7168 6.1 / 8.5; A4W4 1 x 1536 x 12288 5.4 / 8.2; preshuffled
-// bf16 1 x 1536 x 12288 20.3 / 14.0).
+// copied through LDS (MXFP8: 6.3 against 8.8 us at 24 x 1088 x 7168).
+//
+// K is split where its serial walk costs more than the fill and finish launches
+// (about 3 us) do.  us unsplit / split, weights rotated: f32 output, which the
+// splits add up in place (no finish, and shorter chains of roundings: relative
+// error 1.8e-7 / 1.1e-7), 16 x 64 x 4096 9.0 / 5.5, 24 x 256 x 7168 10.2 / 8.5;
+// preshuffled bf16 from K = 7168 (16 x 256 x 4096 6.9 / 7.4, x 7168 10.2 / 8.4);
+// row-major bf16, which has LDS forms, from 14336 (16 x 512 x 7168 7.0 / 9.9, x
+// 14336 11.7 / 10.3), above 16 rows from 12288 (32 x 3072 x 6144 17.2 / 26.8, 32 x
+// 1536 x 12288 30.4 / 26.8); MX from 16384 without an LDS form (A4W4 16 x 512 x
+// 14336 6.3 / 8.1).
 const Instance* skinny_rule(Family f, const Variant& v, int M, int N, int K, int cus, int* splits) {
     const int bm = M <= 16 ? 16 : 32;
     auto pick = [&](int bn, bool split) {
@@ -176,14 +181,15 @@ const Instance* skinny_rule(Family f, const Variant& v, int M, int N, int K, int
     const Instance *n16 = pick(16, false), *n32 = pick(32, false);
     const int blk32 = (N + 31) / 32;
     *splits = 1;
-    if (n32 && (!n16 || (blk32 * 4 >= cus * 3 && (M > 16 || blk32 <= cus)) || (M > 16 && n32->rank > n16->rank)))
-        return n32;
-    const int s = skinny_splits((N + 15) / 16, K / (f == kA16W16 ? 32 : 128), cus, f == kA16W16 ? 128 : 64);
-    if (s > 1 && n16 && n16->rank == 0)
+    const bool bf16 = f == kA16W16, staged = n32 && n16 && M > 16 && n32->rank > n16->rank;
+    const int from = v.out_f32 ? 0 : !bf16 ? 16384 : v.b_pre ? 7168 : M > 16 ? 12288 : 14336;
+    const int s = K < from ? 1 : skinny_splits((N + 15) / 16, K / (bf16 ? 32 : 128), cus);
+    if (s > 1 && (bf16 || v.out_f32 || (n16 && n16->rank == 0 && !staged)))
         if (const Instance* in = pick(16, true)) {
             *splits = s;
             return in;
         }
+    if (n32 && (!n16 || staged || (blk32 * 4 >= cus * 3 && (M > 16 || blk32 <= cus)))) return n32;
     return n16;
 }
 

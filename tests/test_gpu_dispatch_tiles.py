@@ -83,6 +83,31 @@ def test_dispatch_shapes(cuda, fam, m, n, k):
     assert ok, msg
 
 
+# both sides of the K from which up to 32 rows are split, per family and rows
+@pytest.mark.parametrize("fam,m,n,k", [("a16w16_pre", 9, 80, 7104), ("a16w16_pre", 9, 80, 7168), ("a16w16", 32, 80, 12224),
+                                       ("a16w16", 32, 80, 12288), ("a16w16", 16, 80, 12288), ("a16w16", 16, 80, 14336),
+                                       ("a4w4", 7, 80, 16128), ("a4w4", 7, 80, 16384), ("a4w4", 25, 80, 16384),
+                                       ("a8w4", 16, 80, 16384), ("a8w4", 17, 80, 16384)])
+def test_skinny_split_lines(cuda, fam, m, n, k):
+    test_dispatch_shapes(cuda, fam, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 1024), (16, 80, 2048), (17, 80, 2048), (32, 256, 7168)])
+def test_skinny_f32_split_error(cuda, m, n, k):
+    """f32 output up to 32 rows, K split where it is long: the sums stay within a
+    chain of K / 256 f32 roundings (8 waves, 32 products per step) plus the 8 + 8
+    that add the waves and the splits."""
+    from aiter_amd import tgemm
+
+    announce(f"skinny f32 {m}x{n}x{k}")
+    x = torch.randn(m, k, device=cuda, dtype=torch.bfloat16)
+    w = torch.randn(n, k, device=cuda, dtype=torch.bfloat16)
+    got = tgemm.mm(x, w, None, otype=torch.float32).double().cpu()
+    x, w = x.double().cpu(), w.double().cpu()
+    bound = (k / 256 + 16) * 2.0 ** -24 * (x.abs() @ w.abs().t())
+    assert ((got - x @ w.t()).abs() <= bound).all()
+
+
 def test_split_choice_under_capture(cuda):
     """A shape for which the dispatch splits K eagerly: captured on a stream
     without a workspace it runs without the split, and replays give that result."""
