@@ -140,6 +140,8 @@ SIGNATURES = {
     "batched_gemm_bf16_tune": ([_T] * 3 + [ctypes.c_int, ctypes.c_int, _S], ctypes.c_int),
     "aiter_amd_num_kernels": ([], ctypes.c_int),
     "aiter_amd_kernel_info": ([ctypes.c_int, ctypes.c_char_p, ctypes.c_int], ctypes.c_int),
+    "aiter_amd_num_instances": ([], ctypes.c_int),
+    "aiter_amd_instance_info": ([ctypes.c_int, ctypes.c_char_p, ctypes.c_int], ctypes.c_int),
     "aiter_amd_resolve_kernel_name": ([ctypes.c_char_p] + [ctypes.c_int] * 4 + [ctypes.c_int64], ctypes.c_int),
     "aiter_amd_resolve_opus_kid": ([ctypes.c_int, ctypes.c_int, ctypes.c_int64], ctypes.c_int),
     "gemm_workspace_reserve": ([ctypes.c_int, _S, ctypes.c_size_t], ctypes.c_int),
@@ -222,20 +224,32 @@ def call(name: str, *args, device: torch.device | None = None):
         raise RuntimeError(f"{name} failed: {msg.decode() if msg else 'unknown error'}")
 
 
-def kernel_table():
-    """[(id, name, family, skinny, bm, bn, split, a_pre, b_pre, out_f32)] of the library."""
-    l = lib()
+def _table(num, info):
     out = []
     buf = ctypes.create_string_buffer(256)
-    for i in range(l.aiter_amd_num_kernels()):
-        if l.aiter_amd_kernel_info(i, buf, 256) == 0:
+    for i in range(num()):
+        if info(i, buf, 256) == 0:
             f = buf.value.decode().split(",")
             out.append((int(f[0]), f[1], f[2], bool(int(f[3])), int(f[4]), int(f[5]),
                         bool(int(f[6])), bool(int(f[7])), bool(int(f[8])), bool(int(f[9]))))
     return out
 
 
+def kernel_table():
+    """[(id, name, family, skinny, bm, bn, split, a_pre, b_pre, out_f32)] of the library."""
+    l = lib()
+    return _table(l.aiter_amd_num_kernels, l.aiter_amd_kernel_info)
+
+
+@functools.lru_cache(maxsize=1)
+def instance_table() -> tuple:
+    """kernel_table() and after it the instances outside the table (tiles whose
+    row counts are no power of two), which names and the tuner reach as well."""
+    l = lib()
+    return tuple(_table(l.aiter_amd_num_instances, l.aiter_amd_instance_info))
+
+
 @functools.lru_cache(maxsize=1)
 def kernel_names() -> frozenset:
     """Names of this library's kernel instances."""
-    return frozenset(row[1] for row in kernel_table())
+    return frozenset(row[1] for row in instance_table())

@@ -1336,17 +1336,24 @@ int aiter_amd_num_kernels(void) {
     return n;
 }
 
-// Writes "id,name,family,skinny,bm,bn,split,a_pre,b_pre,out_f32" for kernel
-// `id` into buf; returns -1 if id is out of range.
-int aiter_amd_kernel_info(int id, char* buf, int buflen) {
-    const Instance* in = find_by_id(id);
-    if (!in || !in->listed || !buf || buflen <= 0) return -1;
+// "id,name,family,skinny,bm,bn,split,a_pre,b_pre,out_f32" of an instance
+static int write_info(const Instance* in, char* buf, int buflen) {
+    if (!in || !buf || buflen <= 0) return -1;
     static const char* fam[] = {"a4w4", "a8w4", "a16w16"};
     snprintf(buf, buflen, "%d,%s,%s,%d,%d,%d,%d,%d,%d,%d", in->id, in->name.c_str(), fam[in->fam],
              (int)in->skinny, in->bm, in->bn, (int)in->split, (int)in->var.a_pre, (int)in->var.b_pre,
              (int)in->var.out_f32);
     return 0;
 }
+
+// -1 if id is out of range
+int aiter_amd_kernel_info(int id, char* buf, int buflen) {
+    const Instance* in = find_by_id(id);
+    return write_info(in && in->listed ? in : nullptr, buf, buflen);
+}
+
+int aiter_amd_num_instances(void) { return (int)registry().size(); }
+int aiter_amd_instance_info(int id, char* buf, int buflen) { return write_info(find_by_id(id), buf, buflen); }
 
 int aiter_amd_resolve_kernel_name(const char* name, int family, int a_pre, int b_pre, int out_f32, int64_t M) {
     if (!name || !name[0] || family < 0 || family > 2) return -2;

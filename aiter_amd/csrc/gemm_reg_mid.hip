@@ -24,7 +24,7 @@ void RegBuilder::part_mid() {
     AA_MID(kA8W4, "a8w4", kFp8, true, 32, 128, 1, pre)
     AA_MID(kA8W4, "a8w4", kFp8, true, 128, 64, 2, pre)
     tsplit(kA8W4, 128, 128, pre, launch_t32<kFp8, true, 128, 128, 2, false, true>, "a8w4");
-    // row counts that are no power of two: not in the kernel table
+    // row counts that are no power of two: not in the kernel table (its bm are powers of two)
     const size_t unlisted = reg.size();
     AA_MID(kA16W16, "a16w16", kBf16, false, 96, 128, 1, b16r)
     AA_MID(kA16W16, "a16w16", kBf16, false, 160, 128, 1, b16r)

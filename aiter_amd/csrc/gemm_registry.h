@@ -42,7 +42,7 @@ struct Instance {
     int rank = 0;              // among skinny forms of one shape the heuristic takes the highest
     bool stream_k = false;     // skinny stream-K form: one workgroup per CU, partial blocks summed in place
     bool by_ref = true;        // may stand for a reference kernel of the same tile
-    bool listed = true;        // in the kernel table (unlisted instances come last and are run by name or dispatch)
+    bool listed = true;        // in the kernel table (the others come last: aiter_amd_instance_info)
     const struct GemmCost* cost = nullptr;   // time model (gemm_cost.h); null: never the model's choice
 };
 

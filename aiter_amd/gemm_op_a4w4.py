@@ -16,7 +16,7 @@ import torch
 from torch import Tensor
 
 from . import dtypes
-from ._lib import call, kernel_names
+from ._lib import call, instance_table, kernel_names
 from .config import A4W4_KEYS, DEFAULT_A4W4_CSV, get_cu_num, get_gfx, load_tuned, row_kernel, tuned_row
 from .gemm_common import get_padded_m
 
@@ -160,11 +160,9 @@ def gemm_a4w4_blockscale(XQ: Tensor, WQ: Tensor, x_scale: Tensor, w_scale: Tenso
     block shape here, or the heuristic choice when this library has no such
     tile; an empty name the heuristic.  Other names raise, as in the
     reference."""
-    from ._lib import kernel_table
-
     kid = -1
     if kernelName:
-        for row in kernel_table():
+        for row in instance_table():
             if row[1] == kernelName:
                 kid = row[0]
         if kid < 0:

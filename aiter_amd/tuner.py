@@ -45,7 +45,7 @@ import pandas as pd
 import torch
 
 from . import dtypes
-from ._lib import call, kernel_table
+from ._lib import call, instance_table
 from .config import A4W4_COLUMNS, BF16_COLUMNS, get_cu_num, get_gfx
 from .quant import dynamic_mxfp4_quant, dynamic_mxfp8_quant
 from .shuffle import shuffle_weight
@@ -198,7 +198,7 @@ def _copies(per_call_bytes: int) -> int:
 def candidates(family: str, M: int, bpreshuffle: bool = True, out_f32: bool = False):
     """(kernel id, name, log2 split) triples of this library for the shape."""
     out = []
-    for (kid, name, fam, skinny, bm, bn, split, a_pre, b_pre, of32) in kernel_table():
+    for (kid, name, fam, skinny, bm, bn, split, a_pre, b_pre, of32) in instance_table():
         if fam != family or a_pre or b_pre != bpreshuffle or of32 != out_f32:
             continue
         if skinny and M > bm:

@@ -366,6 +366,10 @@ int moe_sum(aiter_tensor_t* input, aiter_tensor_t* output, aiter_stream_t stream
  * "id,name,family,skinny,bm,bn,split,a_pre,b_pre,out_f32" (0 or -1). */
 int aiter_amd_num_kernels(void);
 int aiter_amd_kernel_info(int id, char* buf, int buflen);
+/* The same over every instance that a name or the dispatch can run: the table's
+ * ids, then those of the tiles whose row counts are no power of two. */
+int aiter_amd_num_instances(void);
+int aiter_amd_instance_info(int id, char* buf, int buflen);
 
 /* Tuned-CSV name resolution, the lookup gemm_a4w4_asm / gemm_a16w16_asm /
  * mxfp8_mxfp4_gemm_asm apply to kernelName (the reference resolves names in

@@ -1,0 +1,53 @@
+"""What the dispatch runs for a call, on the CPU: the names it knows, a tuned
+row's kernel, and the instance and split count that the library chooses."""
+import pandas as pd
+import pytest
+import torch
+
+from aiter_amd import fused_gemm, gemm_op_a4w4, tuner
+from aiter_amd._lib import instance_table, kernel_names, kernel_table
+from tests.test_dispatch import _clear, _row, gfx950  # noqa: F401
+
+
+def _unlisted():
+    try:
+        return [r[1] for r in instance_table()[len(kernel_table()):]]
+    except RuntimeError:   # not built
+        return []
+
+
+UNLISTED = _unlisted()
+
+
+def test_instances_outside_the_table():
+    """The 96-, 160- and 192-row tiles follow the kernel table's ids."""
+    assert instance_table()[:len(kernel_table())] == tuple(kernel_table())
+    assert {r[4] for r in instance_table()[len(kernel_table()):]} == {96, 160, 192}
+    assert set(UNLISTED) <= kernel_names()
+
+
+@pytest.mark.parametrize("name", [n for n in UNLISTED if n.startswith("a4w4")])
+def test_row_naming_an_instance_outside_the_table(name, tmp_path, monkeypatch, gfx950):
+    """A caller's row with such a name runs that kernel with the call's bias,
+    alpha and beta (a name the library does not know goes to the CK entry, which
+    has none of them)."""
+    p = tmp_path / "t.csv"
+    pd.DataFrame([_row(300, 512, 512, name, split=1)]).to_csv(p, index=False)
+    monkeypatch.setenv("AITER_CONFIG_GEMM_A4W4", str(p))
+    _clear()
+    seen = []
+    monkeypatch.setattr(gemm_op_a4w4, "call", lambda *a: seen.append(a))
+    a, w = torch.zeros(300, 256, dtype=torch.uint8), torch.zeros(512, 256, dtype=torch.uint8)
+    s = torch.zeros(512, 16, dtype=torch.uint8)
+    bias = torch.ones(512)
+    gemm_op_a4w4.gemm_a4w4(a, w, s, s, bias=bias, alpha=0.5, beta=2.0)
+    (entry, *args), = seen
+    assert entry == "gemm_a4w4_asm"
+    assert args[5] == name and args[6] is bias and args[7:11] == [0.5, 2.0, 1, 1]
+    assert fused_gemm._tuned_a4w4(300, 512, 512, True) == name
+
+
+def test_tuner_sees_every_instance():
+    names = {n for fam in ("a4w4", "a8w4", "a16w16") for pre in (False, True)
+             for _, n, _ in tuner.candidates(fam, 150, pre)}
+    assert set(UNLISTED) <= names
