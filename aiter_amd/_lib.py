@@ -144,6 +144,9 @@ SIGNATURES = {
     "aiter_amd_instance_info": ([ctypes.c_int, ctypes.c_char_p, ctypes.c_int], ctypes.c_int),
     "aiter_amd_resolve_kernel_name": ([ctypes.c_char_p] + [ctypes.c_int] * 4 + [ctypes.c_int64], ctypes.c_int),
     "aiter_amd_resolve_opus_kid": ([ctypes.c_int, ctypes.c_int, ctypes.c_int64], ctypes.c_int),
+    "aiter_amd_gemm_choice": ([ctypes.c_int] * 4 + [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.c_int, ctypes.c_char_p,
+                               ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_char_p, ctypes.c_int],
+                              ctypes.c_int),
     "gemm_workspace_reserve": ([ctypes.c_int, _S, ctypes.c_size_t], ctypes.c_int),
     "aiter_amd_workspace_bytes": ([ctypes.c_int, _S], ctypes.c_int64),
     "aiter_amd_workspace_release": ([ctypes.c_int, _S], ctypes.c_int),
@@ -253,3 +256,15 @@ def instance_table() -> tuple:
 def kernel_names() -> frozenset:
     """Names of this library's kernel instances."""
     return frozenset(row[1] for row in instance_table())
+
+
+def gemm_choice(family: str, M: int, N: int, K: int, kernel_name: str = "", a_pre=False, b_pre=True, out_f32=False,
+                batch: int = 1, bias: bool = False, splits: int = 0, cus: int = 256, held: int = -1):
+    """(kernel name, K splits) that the library runs for such a GEMM (aiter_amd_gemm_choice)."""
+    buf = ctypes.create_string_buffer(256)
+    l = lib()
+    if l.aiter_amd_gemm_choice(("a4w4", "a8w4", "a16w16").index(family), int(a_pre), int(b_pre), int(out_f32), M, N, K,
+                               batch, int(bias), kernel_name.encode(), splits, cus, held, buf, 256) != 0:
+        raise RuntimeError(l.aiter_get_last_error().decode())
+    name, sp = buf.value.decode().split(",")
+    return name, int(sp)

@@ -197,8 +197,8 @@ const Instance* skinny_rule(Family f, const Variant& v, int M, int N, int K, int
 // The instance that the time model puts `sc.margin` or more below `base` with
 // `base_splits` (else base): the model is off by about that much between
 // neighbouring tiles, and without the margin twice as many shapes ran over 5 %
-// slower than by the simple rule.  *splits: the split count of a split tile (0:
-// base).  Splits that need more than `ws_bytes` of partials are left out.
+// slower than by the simple rule.  *splits: the split count of a split tile (1 of
+// others, 0: the base as it is; the base may win with another count).  Splits that need more than `ws_bytes` of partials are left out.
 const Instance* modelled_choice(const Instance* base, int base_splits, int M, int N, int K, int cus,
                                 const ModelScope& sc, size_t ws_bytes, int* splits) {
     const int nst = K / (base->fam == kA16W16 ? 64 : 256);
@@ -485,6 +485,73 @@ struct GemmCall {
     GemmParams* capture = nullptr;
 };
 
+// What a call runs: the instance and, when it is a split form, its K splits
+// (the launcher takes whole stages per split, so it may run fewer).
+struct Choice {
+    const Instance* inst = nullptr;
+    int splits = 1;
+};
+
+// The instance of a call: the named one, that of a reference kernel's tile, or
+// the dispatch's own.  room(): bytes of partials that the call's stream may use.
+template <typename Room>
+Choice choose(const GemmCall& c, int M, int N, int K, bool bias, int cus, Room&& room) {
+    const bool scaled = c.fam != kA16W16, batched = c.batch > 1;
+    const int nst = K / (scaled ? 256 : 64);
+    // "~name": the choice of a tuned row for other row counts, which the time
+    // model may replace
+    const char* name = c.kernel_name && c.kernel_name[0] ? c.kernel_name : nullptr;
+    const bool hint = name && name[0] == '~';
+    if (hint) ++name;
+    const Instance* inst = nullptr;
+    if (c.kernel_id >= 0) {
+        inst = find_by_id(c.kernel_id);
+        AA_CHECK(inst && variant_ok(*inst, c.fam, c.var), "kernel id ", c.kernel_id, " does not fit this GEMM");
+    } else if (name) {
+        bool known = false;
+        inst = resolve_name(name, c.fam, c.var, M, &known);
+        AA_CHECK(known, "unknown kernel name '", name, "'");
+        if (inst) AA_CHECK(variant_ok(*inst, c.fam, c.var), "kernel '", name, "' does not fit this GEMM");
+    } else if (c.ref_tile.tm > 0) {
+        inst = reference_tile_instance(c.ref_tile, c.fam, c.var, M);
+    }
+    // requested split count (0: none)
+    const int req_splits =
+        c.split_count > 0 ? c.split_count : (c.log2_split >= 0 ? 1 << std::min(c.log2_split, 16) : 0);
+    const bool named = inst != nullptr;
+    int splits = 1;
+    if (!named) {
+        inst = simple_rule(c.fam, c.var, M, N, K, cus, &splits);
+        AA_CHECK(inst, "no kernel instance for this GEMM");
+    } else if (inst->skinny && inst->split) {
+        splits = skinny_splits((N + 15) / 16, K / (scaled ? 128 : 32), cus);
+    }
+    if (!inst->split) splits = 1;
+    else if (req_splits > 0) splits = req_splits;
+    else if (!inst->skinny) splits = tile_splits(((M + inst->bm - 1) / inst->bm) * ((N + inst->bn - 1) / inst->bn), nst, cus);
+    if (!(hint || (!named && req_splits == 0)) || M <= 16 || !inst->cost) return {inst, splits};
+
+    ModelScope sc;
+    sc.batch = c.batch;
+    // a tuned row's tile was the best of all at its own row count: gains
+    // modelled below 8 % measured as ties (bf16 1573 x 14336 x 4096 179.5 us
+    // by the row, 180.1 by the model; 150 x 14336 x 4096 34.7 / 35.2)
+    if (hint) sc.margin = 1.08f;
+    sc.persistent = !batched && !bias && !c.epi.kind;
+    const int have = batched ? 1 : !inst->split || inst->skinny ? splits : tile_split_count(*inst, M, N, K, cus, splits);
+    int sp = 0;
+    const Instance* best =
+        modelled_choice(inst, have, M, N, K, cus, sc, c.scratch ? c.scratch_bytes : ~size_t(0), &sp);
+    if (best->split && sp > 0 && !c.scratch) {
+        // under graph capture the workspace cannot grow
+        const size_t limit = room();
+        if ((size_t)sp * M * N * sizeof(float) > limit)
+            best = modelled_choice(inst, have, M, N, K, cus, sc, limit, &sp);
+    }
+    // sp 0: the base as it is
+    return sp > 0 ? Choice{best, sp} : Choice{inst, splits};
+}
+
 // split-K partial buffer of a call: the call's scratch when it brings one
 // (never grown: too small is an error), else the (device, stream) workspace
 float* split_buffer(const GemmCall& c, int dev, hipStream_t st, size_t need) {
@@ -640,70 +707,17 @@ void run_gemm(const GemmCall& c, hipStream_t stream) {
     if (dev < 0) AA_HIP(hipGetDevice(&dev));
     const int cus = device_cu_count(dev);
 
-    const Instance* inst = nullptr;
     p.bs_a = c.bs_a;
     p.bs_b = c.bs_b;
     p.bs_d = c.bs_d;
     p.bs_bias = c.bs_bias;
     AA_CHECK(c.batch >= 1 && c.batch < 65536, "batch must be in [1, 65535]");
     const bool batched = c.batch > 1;   // one-pass, one-tile-per-workgroup kernels only
-    int splits = 1;
-    // "~name": the choice of a tuned row for other row counts, which the time
-    // model may replace
-    const char* name = c.kernel_name && c.kernel_name[0] ? c.kernel_name : nullptr;
-    const bool hint = name && name[0] == '~';
-    if (hint) ++name;
-    if (c.kernel_id >= 0) {
-        inst = find_by_id(c.kernel_id);
-        AA_CHECK(inst && variant_ok(*inst, c.fam, c.var), "kernel id ", c.kernel_id, " does not fit this GEMM");
-    } else if (name) {
-        bool known = false;
-        inst = resolve_name(name, c.fam, c.var, M, &known);
-        AA_CHECK(known, "unknown kernel name '", name, "'");
-        if (inst) AA_CHECK(variant_ok(*inst, c.fam, c.var), "kernel '", name, "' does not fit this GEMM");
-    } else if (c.ref_tile.tm > 0) {
-        inst = reference_tile_instance(c.ref_tile, c.fam, c.var, M);
-    }
     const int ksteps = (int)(K / (scaled ? 128 : 32));
-    // requested split count (0: the launcher chooses); the model's (0: none)
-    int req_splits = c.split_count > 0 ? c.split_count : (c.log2_split >= 0 ? 1 << std::min(c.log2_split, 16) : 0);
-    int auto_splits = 0;
-    const bool named = inst != nullptr;
-    if (!inst) {
-        inst = simple_rule(c.fam, c.var, (int)M, (int)N, (int)K, cus, &auto_splits);
-        AA_CHECK(inst, "no kernel instance for this GEMM");
-        if (inst->skinny && inst->split) splits = auto_splits;
-    } else if (inst->skinny && inst->split) {
-        splits = skinny_splits((int)((N + 15) / 16), ksteps, cus);
-    }
-    if ((hint || (!named && req_splits == 0)) && M > 16 && inst->cost) {
-        ModelScope sc;
-        sc.batch = c.batch;
-        // a tuned row's tile was the best of all at its own row count: gains
-        // modelled below 8 % measured as ties (bf16 1573 x 14336 x 4096 179.5 us
-        // by the row, 180.1 by the model; 150 x 14336 x 4096 34.7 / 35.2)
-        if (hint) sc.margin = 1.08f;
-        sc.persistent = !batched && !p.bias && !c.epi.kind;
-        const int have = !inst->split || inst->skinny ? splits
-                         : batched                    ? 1
-                                                      : tile_split_count(*inst, (int)M, (int)N, (int)K, cus, req_splits);
-        int sp = 0;
-        const Instance* best =
-            modelled_choice(inst, have, (int)M, (int)N, (int)K, cus, sc, c.scratch ? c.scratch_bytes : ~size_t(0), &sp);
-        if (best != inst && best->split && !c.scratch) {
-            // under graph capture the workspace cannot grow
-            const size_t room = workspace_limit(dev, stream);
-            if ((size_t)sp * M * N * sizeof(float) > room)
-                best = modelled_choice(inst, have, (int)M, (int)N, (int)K, cus, sc, room, &sp);
-        }
-        if (best != inst) {
-            inst = best;
-            auto_splits = sp;
-            req_splits = 0;
-            splits = 1;
-        }
-    }
-    if (inst->skinny && inst->split && req_splits > 0) splits = req_splits;
+    const Choice choice =
+        choose(c, (int)M, (int)N, (int)K, p.bias != nullptr, cus, [&] { return workspace_limit(dev, stream); });
+    const Instance* inst = choice.inst;
+    int splits = choice.splits;
     if (inst->skinny) AA_CHECK(M <= inst->bm, "skinny kernel ", inst->name, " covers M <= ", inst->bm);
     AA_CHECK(!c.capture || (inst->skinny && !inst->split && !inst->stream_k && !batched),
              "planned calls take non-split skinny kernels");
@@ -716,9 +730,7 @@ void run_gemm(const GemmCall& c, hipStream_t stream) {
         if (inst->split) {
             // split-K tile: stages of K over gridDim.y, f32 slices, then a sum
             const int nst = (int)(K / (scaled ? 256 : 64));
-            int sp = req_splits > 0 ? req_splits : auto_splits > 0 ? auto_splits : tile_splits(tiles, nst, cus);
-            if (batched) sp = 1;
-            sp = std::max(1, std::min(sp, nst));
+            int sp = batched ? 1 : std::max(1, std::min(splits, nst));
             p.k_steps_per_split = (nst + sp - 1) / sp;
             sp = (nst + p.k_steps_per_split - 1) / p.k_steps_per_split;
             if (sp > 1) {
@@ -1360,6 +1372,22 @@ int aiter_amd_resolve_kernel_name(const char* name, int family, int a_pre, int b
     bool known = false;
     const Instance* in = resolve_name(name, (Family)family, Variant{a_pre != 0, b_pre != 0, out_f32 != 0}, M, &known);
     return !known ? -2 : (in ? in->id : -1);
+}
+
+int aiter_amd_gemm_choice(int family, int a_pre, int b_pre, int out_f32, int64_t M, int64_t N, int64_t K, int batch,
+                          int bias, const char* kernelName, int splits, int cus, int64_t held, char* buf, int buflen) {
+    return safe_call([&] {
+        AA_CHECK(family >= 0 && family <= 2 && M > 0 && N > 0 && K > 0 && batch > 0 && cus > 0 && buf && buflen > 0 &&
+                     M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31),
+                 "aiter_amd_gemm_choice: arguments out of range");
+        GemmCall c{(Family)family, Variant{a_pre != 0, b_pre != 0, out_f32 != 0}, nullptr, nullptr, nullptr, nullptr,
+                   nullptr, nullptr, 1.0f, 0.0f, kernelName, -1, -1};
+        c.split_count = splits;
+        c.batch = batch;
+        const Choice ch = choose(c, (int)M, (int)N, (int)K, bias != 0, cus,
+                                 [&] { return held < 0 ? ~size_t(0) : (size_t)held; });
+        snprintf(buf, buflen, "%s,%d", ch.inst->name.c_str(), ch.splits);
+    });
 }
 
 int aiter_amd_resolve_opus_kid(int kid, int out_f32, int64_t M) {

@@ -382,6 +382,12 @@ int aiter_amd_instance_info(int id, char* buf, int buflen);
  * (row-major B).  No GPU call. */
 int aiter_amd_resolve_kernel_name(const char* name, int family, int a_pre, int b_pre, int out_f32, int64_t M);
 int aiter_amd_resolve_opus_kid(int kid, int out_f32, int64_t M);
+/* The kernel that a GEMM call of these sizes runs on a GPU of `cus` CUs, written
+ * as "name,K splits": kernelName ("" or NULL: the library's choice) and splits
+ * (a literal request, 0: none) as in the GEMM entries, held the workspace bytes
+ * of a captured call's stream (negative: not captured).  No GPU call. */
+int aiter_amd_gemm_choice(int family, int a_pre, int b_pre, int out_f32, int64_t M, int64_t N, int64_t K, int batch,
+                          int bias, const char* kernelName, int splits, int cus, int64_t held, char* buf, int buflen);
 
 /* Pre-sizes the split-K fp32 workspace owned by (device, stream) to at least
  * `bytes` (and allocates its split-K tile counters, 64K of them), so that a

@@ -1,0 +1,38 @@
+"""The choices of the dispatch as the GPU runs them: split counts through the
+workspace that a call leaves, and results against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from aiter_amd._lib import call, gemm_choice, lib
+from oracle import mx_oracle as O
+from tests.conftest import announce
+from tests.mx_inputs import allclose_report, bf16_operand
+
+pytestmark = pytest.mark.gpu
+
+
+def _bf16_case(m, n, k, cuda, shuffled):
+    a, b = bf16_operand(m, k, 5), bf16_operand(n, k, 6)
+    ref = O.bf16_bits_to_f32(O.gemm_a16w16_ref(a, b))
+    w = O.shuffle_weight(b) if shuffled else b
+    A, B = (torch.from_numpy(v.view(np.int16).copy()).to(cuda).view(torch.bfloat16) for v in (a, w))
+    return A, B, ref
+
+
+@pytest.mark.parametrize("m,n,k", [(43, 512, 3904), (70, 256, 4096)])
+def test_choice_is_what_runs(cuda, m, n, k):
+    """A split choice leaves its partials' bytes in a released stream's workspace."""
+    announce(f"dispatch choice {m}x{n}x{k}")
+    name, splits = gemm_choice("a16w16", m, n, k)
+    assert "splitk" in name and splits > 1
+    A, B, ref = _bf16_case(m, n, k, cuda, True)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=cuda)
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        assert lib().aiter_amd_workspace_release(0, st.cuda_stream) == 0
+        call("gemm_a16w16_asm", A, B, out, None, None, 0, None, 1)
+    torch.cuda.synchronize()
+    assert lib().aiter_amd_workspace_bytes(0, st.cuda_stream) == splits * m * n * 4
+    ok, msg = allclose_report(out.float().cpu().numpy(), ref)
+    assert ok, msg

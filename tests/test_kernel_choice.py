@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from aiter_amd import fused_gemm, gemm_op_a4w4, tuner
-from aiter_amd._lib import instance_table, kernel_names, kernel_table
+from aiter_amd._lib import gemm_choice, instance_table, kernel_names, kernel_table
 from tests.test_dispatch import _clear, _row, gfx950  # noqa: F401
 
 
@@ -51,3 +51,12 @@ def test_tuner_sees_every_instance():
     names = {n for fam in ("a4w4", "a8w4", "a16w16") for pre in (False, True)
              for _, n, _ in tuner.candidates(fam, 150, pre)}
     assert set(UNLISTED) <= names
+
+
+@pytest.mark.parametrize("fam,m,n,k", [("a16w16", 43, 512, 3904), ("a8w4", 36, 2064, 15616)])
+def test_more_splits_of_the_base_instance(fam, m, n, k):
+    """The time model's answer may be the simple rule's own split tile with
+    another count: here 8 splits, where the rule's count is 4."""
+    name, splits = gemm_choice(fam, m, n, k)
+    assert "splitk" in name and splits == 8
+    assert gemm_choice(fam, m, n, k, kernel_name=name)[1] == 4   # by name: the launcher's own count
