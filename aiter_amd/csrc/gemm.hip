@@ -442,8 +442,8 @@ float* workspace(int dev, hipStream_t st, size_t bytes, int slot = 0) {
     return w.ptr;
 }
 
-// Partials that a call on `st` may put into the workspace: no limit, but under
-// graph capture what is there already (it cannot grow then).
+// Bytes that the workspace of `st` can hold: no limit, but under graph capture
+// what is there already (it cannot grow then).
 size_t workspace_limit(int dev, hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     AA_HIP(hipStreamIsCapturing(st, &cs));
@@ -492,8 +492,15 @@ struct Choice {
     int splits = 1;
 };
 
+// Partials that a modelled split may ask for beyond the base's own: 64 MiB,
+// 256 KiB per CU, which the simple rule's splits reach as well (one 256x256 f32
+// tile per CU).  One reservation of that size covers every choice of a stream.
+constexpr size_t kChoiceWorkspaceBytes = size_t(64) << 20;
+
 // The instance of a call: the named one, that of a reference kernel's tile, or
-// the dispatch's own.  room(): bytes of partials that the call's stream may use.
+// the dispatch's own.  room(): bytes that the workspace of the call's stream can
+// hold.  A captured call whose choice needs more than that (no reservation) takes
+// one that needs no more than the base, whatever else the stream holds.
 template <typename Room>
 Choice choose(const GemmCall& c, int M, int N, int K, bool bias, int cus, Room&& room) {
     const bool scaled = c.fam != kA16W16, batched = c.batch > 1;
@@ -539,15 +546,12 @@ Choice choose(const GemmCall& c, int M, int N, int K, bool bias, int cus, Room&&
     if (hint) sc.margin = 1.08f;
     sc.persistent = !batched && !bias && !c.epi.kind;
     const int have = batched ? 1 : !inst->split || inst->skinny ? splits : tile_split_count(*inst, M, N, K, cus, splits);
+    const size_t slice = (size_t)M * N * sizeof(float), base_need = have > 1 ? have * slice : 0;
     int sp = 0;
-    const Instance* best =
-        modelled_choice(inst, have, M, N, K, cus, sc, c.scratch ? c.scratch_bytes : ~size_t(0), &sp);
-    if (best->split && sp > 0 && !c.scratch) {
-        // under graph capture the workspace cannot grow
-        const size_t limit = room();
-        if ((size_t)sp * M * N * sizeof(float) > limit)
-            best = modelled_choice(inst, have, M, N, K, cus, sc, limit, &sp);
-    }
+    const Instance* best = modelled_choice(inst, have, M, N, K, cus, sc,
+                                           c.scratch ? c.scratch_bytes : std::max(base_need, kChoiceWorkspaceBytes), &sp);
+    if (best->split && sp > 0 && !c.scratch && sp * slice > room())
+        best = modelled_choice(inst, have, M, N, K, cus, sc, base_need, &sp);
     // sp 0: the base as it is
     return sp > 0 ? Choice{best, sp} : Choice{inst, splits};
 }

@@ -391,7 +391,11 @@ int aiter_amd_gemm_choice(int family, int a_pre, int b_pre, int out_f32, int64_t
 
 /* Pre-sizes the split-K fp32 workspace owned by (device, stream) to at least
  * `bytes` (and allocates its split-K tile counters, 64K of them), so that a
- * later HIP-graph capture never needs to allocate.  The
+ * later HIP-graph capture never needs to allocate.  64 MiB cover every split
+ * that the library chooses by itself (a named split kernel takes 4 * splits * M
+ * * N bytes): captured calls then run the kernels that eager ones run.  Without
+ * the bytes, a captured call for which a split is only the faster form takes one
+ * that needs none, and any other split call returns -1.  The
  * reference's counterpart is the caller-provided semaphore / workspace
  * tensor of csrc/py_itfs_cu/asm_gemm_a16w16.cu:192-205 and
  * aiter/ops/opus/gemm_op_opus.py (opus_gemm_workspace_init). */

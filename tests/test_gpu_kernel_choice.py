@@ -36,3 +36,50 @@ def test_choice_is_what_runs(cuda, m, n, k):
     assert lib().aiter_amd_workspace_bytes(0, st.cuda_stream) == splits * m * n * 4
     ok, msg = allclose_report(out.float().cpu().numpy(), ref)
     assert ok, msg
+
+
+def test_reserved_capture_runs_the_eager_kernel(cuda):
+    """With 64 MiB reserved a captured call runs the split that the eager call
+    runs, bit for bit; the same call captured with a few bytes held runs the form
+    without a workspace that it runs with none."""
+    import aiter_amd
+
+    m, n, k = 150, 4096, 14336
+    announce(f"captured choice {m}x{n}x{k}")
+    assert gemm_choice("a16w16", m, n, k, b_pre=False)[1] > 1
+    A, B, ref = _bf16_case(m, n, k, cuda, False)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=cuda)
+    st = torch.cuda.Stream()
+
+    def run():
+        call("gemm_a16w16_asm", A, B, out, None, None, 0, None, 0)
+        return out
+
+    def captured(prepare):
+        with torch.cuda.stream(st):
+            assert lib().aiter_amd_workspace_release(0, st.cuda_stream) == 0
+            prepare()
+            st.synchronize()
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=st):
+                run()
+            res = []
+            for _ in range(3):
+                out.fill_(float("nan"))
+                g.replay()
+                st.synchronize()
+                res.append(out.clone())
+        torch.cuda.synchronize()
+        assert all(torch.equal(r, res[0]) for r in res)
+        return res[0]
+
+    with torch.cuda.stream(st):
+        eager = run().clone()
+    reserved = captured(aiter_amd.opus_gemm_workspace_init)
+    assert torch.equal(reserved, eager)
+    none = captured(lambda: None)
+    few = captured(lambda: lib().gemm_workspace_reserve(0, st.cuda_stream, 4 * m * n * 4))
+    assert torch.equal(none, few)
+    for got in (eager, none):
+        ok, msg = allclose_report(got.float().cpu().numpy(), ref)
+        assert ok, msg

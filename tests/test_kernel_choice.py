@@ -1,5 +1,8 @@
 """What the dispatch runs for a call, on the CPU: the names it knows, a tuned
 row's kernel, and the instance and split count that the library chooses."""
+import math
+import random
+
 import pandas as pd
 import pytest
 import torch
@@ -60,3 +63,39 @@ def test_more_splits_of_the_base_instance(fam, m, n, k):
     name, splits = gemm_choice(fam, m, n, k)
     assert "splitk" in name and splits == 8
     assert gemm_choice(fam, m, n, k, kernel_name=name)[1] == 4   # by name: the launcher's own count
+
+
+def _shapes(n=400, seed=3):
+    rng = random.Random(seed)
+    log_int = lambda lo, hi, step: max(step, int(math.exp(rng.uniform(math.log(lo), math.log(hi)))) // step * step)
+    for i in range(n):
+        fam, kw = [("a16w16", {"b_pre": False}), ("a16w16", {}), ("a4w4", {}), ("a8w4", {})][i % 4]
+        yield fam, kw, log_int(17, 4096, 1), log_int(64, 16384, 16), log_int(512, 28672, 256)
+
+
+def _base(fam, m, n, k, kw):
+    """(name, splits) of the simple rule, which a call with a split request takes as it is"""
+    name = gemm_choice(fam, m, n, k, splits=1, **kw)[0]
+    return name, gemm_choice(fam, m, n, k, kernel_name=name, **kw)[1] if "splitk" in name else 1
+
+
+def test_workspace_of_a_choice():
+    """Eagerly a choice asks for 64 MiB of partials at most (or what the simple
+    rule asks for).  Under capture it is the eager one if the stream holds its
+    bytes; otherwise one that needs no more than the simple rule's, and the same
+    whatever the stream holds."""
+    changed = 0
+    for fam, kw, m, n, k in [("a16w16", {"b_pre": False}, 896, 5488, 27968), *_shapes()]:
+        need = lambda c: c[1] * m * n * 4 if "splitk" in c[0] and c[1] > 1 else 0
+        base = need(_base(fam, m, n, k, kw)) if m > 32 else 0
+        eager = gemm_choice(fam, m, n, k, **kw)
+        if "skinny" in eager[0]:
+            continue
+        assert need(eager) <= max(base, 64 << 20)
+        assert gemm_choice(fam, m, n, k, held=max(base, 64 << 20), **kw) == eager
+        assert gemm_choice(fam, m, n, k, held=need(eager), **kw) == eager
+        if need(eager):
+            others = {gemm_choice(fam, m, n, k, held=h, **kw) for h in (0, need(eager) // 2, need(eager) - 1)}
+            assert len(others) == 1 and need(others.pop()) <= base
+            changed += 1
+    assert changed > 40
