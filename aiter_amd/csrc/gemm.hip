@@ -408,6 +408,8 @@ constexpr int kCounterSlot = 5;
 struct WsVal {
     float* ptr = nullptr;
     size_t bytes = 0;
+    bool captured = false;          // a graph holds `ptr`
+    std::vector<float*> retired;    // outgrown blocks that graphs hold
 };
 
 std::mutex& workspace_mutex() {
@@ -419,35 +421,47 @@ std::map<WsKey, WsVal>& workspace_map() {
     return ws;
 }
 
+bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (st) AA_HIP(hipStreamIsCapturing(st, &cs));   // the null stream is never captured
+    return cs != hipStreamCaptureStatusNone;
+}
+
+// A block that a graph was captured with stays until the stream's workspaces are
+// released: the graph writes to it on every replay, also after a later call has
+// outgrown it.
 float* workspace(int dev, hipStream_t st, size_t bytes, int slot = 0) {
     std::lock_guard<std::mutex> lk(workspace_mutex());
     auto& ws = workspace_map();
+    const bool cap = capturing(st);
     WsVal& w = ws[{dev, st, slot}];
     if (w.bytes < bytes) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        AA_HIP(hipStreamIsCapturing(st, &cs));
-        AA_CHECK(cs == hipStreamCaptureStatusNone, "library workspace slot ", slot,
+        AA_CHECK(!cap, "library workspace slot ", slot,
                  " must be sized before graph capture (split-K: gemm_workspace_reserve; low-precision outputs: "
                  "one eager call of the same shape)");
-        if (w.ptr) {
+        if (w.ptr && w.captured) {
+            w.retired.push_back(w.ptr);
+        } else if (w.ptr) {
             AA_HIP(hipStreamSynchronize(st));
             AA_HIP(hipFree(w.ptr));
         }
+        w.ptr = nullptr;
+        w.bytes = 0;
+        w.captured = false;
         AA_HIP(hipMalloc(&w.ptr, bytes));
         w.bytes = bytes;
         // counters start at zero; their users set them back to zero (never
         // during graph capture: allocation is refused there)
         if (slot == kCounterSlot) AA_HIP(hipMemsetAsync(w.ptr, 0, bytes, st));
     }
+    w.captured |= cap;
     return w.ptr;
 }
 
 // Bytes that the workspace of `st` can hold: no limit, but under graph capture
 // what is there already (it cannot grow then).
 size_t workspace_limit(int dev, hipStream_t st) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    AA_HIP(hipStreamIsCapturing(st, &cs));
-    if (cs == hipStreamCaptureStatusNone) return ~size_t(0);
+    if (!capturing(st)) return ~size_t(0);
     std::lock_guard<std::mutex> lk(workspace_mutex());
     auto it = workspace_map().find({dev, st, 0});
     return it == workspace_map().end() ? 0 : it->second.bytes;
@@ -1553,23 +1567,21 @@ int64_t aiter_amd_workspace_bytes(int device, aiter_stream_t stream) {
     return it == ws.end() ? 0 : (int64_t)it->second.bytes;
 }
 
-// Frees every library workspace held for (device, stream) after the
-// stream's work completes; the next call that needs one allocates it again.
+// Frees every library workspace held for (device, stream), with the blocks that
+// graphs captured on it write to, after the stream's work completes; the next
+// call that needs one allocates it again.
 int aiter_amd_workspace_release(int device, aiter_stream_t stream) {
     return safe_call([&] {
         DeviceGuard g(device);
         hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        AA_HIP(hipStreamIsCapturing(st, &cs));
-        AA_CHECK(cs == hipStreamCaptureStatusNone, "workspaces cannot be released during graph capture");
+        AA_CHECK(!capturing(st), "workspaces cannot be released during graph capture");
         std::lock_guard<std::mutex> lk(workspace_mutex());
         auto& ws = workspace_map();
         for (auto it = ws.begin(); it != ws.end();) {
             if (it->first.dev == device && it->first.st == st) {
-                if (it->second.ptr) {
-                    AA_HIP(hipStreamSynchronize(st));
-                    AA_HIP(hipFree(it->second.ptr));
-                }
+                AA_HIP(hipStreamSynchronize(st));
+                for (float* old : it->second.retired) AA_HIP(hipFree(old));
+                if (it->second.ptr) AA_HIP(hipFree(it->second.ptr));
                 it = ws.erase(it);
             } else {
                 ++it;

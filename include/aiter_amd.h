@@ -408,7 +408,10 @@ int64_t aiter_amd_workspace_bytes(int device, aiter_stream_t stream);
 
 /* No counterpart in the reference: frees every library workspace held for
  * (device, stream) once the stream's queued work has completed (a later call
- * that needs one allocates it again).  Not allowed during graph capture.
+ * that needs one allocates it again), also those that graphs captured on the
+ * stream write to: such graphs must not be replayed afterwards.  Until then a
+ * block that a graph holds stays, also when a later call outgrows it.  Not allowed
+ * during graph capture.
  * Returns 0 or -1 (message in aiter_get_last_error). */
 int aiter_amd_workspace_release(int device, aiter_stream_t stream);
 

@@ -83,3 +83,37 @@ def test_reserved_capture_runs_the_eager_kernel(cuda):
     for got in (eager, none):
         ok, msg = allclose_report(got.float().cpu().numpy(), ref)
         assert ok, msg
+
+
+def test_graph_keeps_the_workspace_it_was_captured_with(cuda):
+    """A larger split call on the stream gets another block; the graph's replays
+    still write to theirs, whatever has been allocated since."""
+    m, n, k = 64, 1024, 1280
+    announce(f"captured workspace outgrown {m}x{n}x{k}")
+    A, B, _ = _bf16_case(m, n, k, cuda, False)
+    big = [t.repeat(8, 1) for t in (A, B)]
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=cuda)
+    out_big = torch.empty((8 * m, 8 * n), dtype=torch.bfloat16, device=cuda)
+    st = torch.cuda.Stream()
+    name = "a16w16_tile_64x64_splitk_bplain"
+    with torch.cuda.stream(st):
+        assert lib().aiter_amd_workspace_release(0, st.cuda_stream) == 0
+        call("gemm_a16w16_asm", A, B, out, None, None, 4, name, 0)
+        eager = out.clone()
+        st.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            call("gemm_a16w16_asm", A, B, out, None, None, 4, name, 0)
+        held = lib().aiter_amd_workspace_bytes(0, st.cuda_stream)
+        call("gemm_a16w16_asm", *big, out_big, None, None, 4, name, 0)
+        assert lib().aiter_amd_workspace_bytes(0, st.cuda_stream) == 64 * held
+        other = [torch.full((held // 4,), 7.0, device=cuda) for _ in range(16)]
+        for _ in range(3):
+            out.fill_(float("nan"))
+            g.replay()
+            st.synchronize()
+            assert torch.equal(out, eager)
+        assert all(bool((t == 7.0).all()) for t in other)
+    torch.cuda.synchronize()
+    assert torch.equal(out_big[:m, :n], eager)
+    assert lib().aiter_amd_workspace_release(0, st.cuda_stream) == 0
