@@ -194,21 +194,33 @@ const Instance* skinny_rule(Family f, const Variant& v, int M, int N, int K, int
     return n16;
 }
 
+// K that one wave's f32 accumulators sum in a row: the waves of a skinny
+// workgroup share K.
+int chain_stages(const Instance& in, int nst, int splits) {
+    const int per = (nst + splits - 1) / splits;
+    return in.skinny ? (per + kSkinnyWaves - 1) / kSkinnyWaves : per;
+}
+
 // The instance that the time model puts `sc.margin` or more below `base` with
 // `base_splits` (else base): the model is off by about that much between
 // neighbouring tiles, and without the margin twice as many shapes ran over 5 %
 // slower than by the simple rule.  *splits: the split count of a split tile (1 of
-// others, 0: the base as it is; the base may win with another count).  Splits that need more than `ws_bytes` of partials are left out.
+// others, 0: the base as it is; the base may win with another count).  Left out:
+// splits that need more than `ws_bytes` of partials, and for f32 outputs whatever
+// sums K in longer chains than the base, whose roundings are the result's error
+// (4009 x 128 x 1472, 2 splits / unsplit: 1.55e-7 / 2.25e-7 against 64 bits).
 const Instance* modelled_choice(const Instance* base, int base_splits, int M, int N, int K, int cus,
                                 const ModelScope& sc, size_t ws_bytes, int* splits) {
     const int nst = K / (base->fam == kA16W16 ? 64 : 256);
     const Instance* best = base;
     float best_us = model_us(*base, M, N, K, base_splits, sc.batch, cus) / sc.margin;
     *splits = 0;
+    const int chain = base->var.out_f32 ? chain_stages(*base, nst, base_splits) : nst;
     for (const Instance* in : modelled(base->fam, base->var)) {
         if (in->persistent && !sc.persistent) continue;
         if (in->skinny && (M > in->bm || M * 2 <= in->bm)) continue;
         if (!in->split) {
+            if (chain_stages(*in, nst, 1) > chain) continue;
             const float us = model_us(*in, M, N, K, 1, sc.batch, cus);
             if (us < best_us) best = in, best_us = us, *splits = 1;
             continue;
@@ -216,7 +228,7 @@ const Instance* modelled_choice(const Instance* base, int base_splits, int M, in
         if (sc.batch > 1) continue;
         for (int want = 2; want <= 8 && nst / want >= 4; want *= 2) {
             const int sp = tile_split_count(*in, M, N, K, cus, want);
-            if (sp < 2 || (size_t)sp * M * N * sizeof(float) > ws_bytes) continue;
+            if (sp < 2 || (size_t)sp * M * N * sizeof(float) > ws_bytes || chain_stages(*in, nst, sp) > chain) continue;
             const float us = model_us(*in, M, N, K, sp, 1, cus);
             if (us < best_us) best = in, best_us = us, *splits = sp;
         }

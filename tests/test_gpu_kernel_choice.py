@@ -117,3 +117,25 @@ def test_graph_keeps_the_workspace_it_was_captured_with(cuda):
     torch.cuda.synchronize()
     assert torch.equal(out_big[:m, :n], eager)
     assert lib().aiter_amd_workspace_release(0, st.cuda_stream) == 0
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 512, 3904), (100, 128, 1024), (1500, 256, 1984), (4009, 128, 1472)])
+def test_f32_error_above_32_rows(cuda, m, n, k):
+    """f32 output: the error of the dispatch's choice is that of the simple
+    rule's kernel, whose chains of f32 roundings it may not exceed (2 % for the
+    roundings' signs, over some thousand outputs)."""
+    from aiter_amd import tgemm
+
+    announce(f"f32 error {m}x{n}x{k}")
+    kw = {"b_pre": False, "out_f32": True}
+    base = gemm_choice("a16w16", m, n, k, splits=1, **kw)[0]
+    splits = gemm_choice("a16w16", m, n, k, kernel_name=base, **kw)[1]
+    x = torch.randn(m, k, device=cuda, dtype=torch.bfloat16)
+    w = torch.randn(n, k, device=cuda, dtype=torch.bfloat16)
+    ref = x.double().cpu() @ w.double().cpu().t()
+    out = torch.empty((m, n), dtype=torch.float32, device=cuda)
+    call("gemm_a16w16_asm", x, w, out, None, None, splits if "splitk" in base else 0, base, 0)
+    err = lambda got: ((got.double().cpu() - ref).norm() / ref.norm()).item()
+    by_rule, by_choice = err(out), err(tgemm.mm(x, w, None, otype=torch.float32))
+    print(f"[error] {by_rule:.3g} {base} x{splits}, {by_choice:.3g} {gemm_choice('a16w16', m, n, k, **kw)}", flush=True)
+    assert by_choice <= 1.02 * by_rule

@@ -99,3 +99,26 @@ def test_workspace_of_a_choice():
             assert len(others) == 1 and need(others.pop()) <= base
             changed += 1
     assert changed > 40
+
+
+def _chain(choice, k):
+    """K that one f32 accumulator sums in a row (the 8 waves of a skinny kernel share K)"""
+    stages = -(-(k // 64) // choice[1])
+    return -(-stages // 8) if "skinny" in choice[0] else stages
+
+
+def test_f32_chains_are_no_longer_than_the_simple_rules():
+    """f32 outputs: no choice sums K in longer chains than the simple rule's."""
+    log_int = lambda rng, lo, hi, step: max(step, int(math.exp(rng.uniform(math.log(lo), math.log(hi)))) // step * step)
+    rng = random.Random(9)
+    shapes = [(4009, 128, 1472)] + [(log_int(rng, 17, 4096, 1), log_int(rng, 32, 512, 16), log_int(rng, 1024, 8192, 64))
+                                    for _ in range(400)]
+    for m, n, k in shapes:
+        for pre in (False, True):
+            kw = {"b_pre": pre, "out_f32": True}
+            base = gemm_choice("a16w16", m, n, k, splits=1, **kw)[0]
+            base = gemm_choice("a16w16", m, n, k, kernel_name=base, **kw)
+            choice = gemm_choice("a16w16", m, n, k, **kw)
+            if "splitk" in choice[0] and "skinny" in choice[0]:
+                continue   # the skinny rule's own split
+            assert _chain(choice, k) <= _chain(base, k), (m, n, k, base, choice)
