@@ -17,6 +17,11 @@
 // shape the dispatch's choice (modelled_choice(), gemm.hip) is 3.5 % (bf16), 2.5 %
 // (A4W4) and 2 % (A8W4) slower on average; by the simple rule alone it would
 // be 11-12 %, 8 % and 8 %.
+//
+// bf16 has no entries up to 32 rows: there the model's choices ran 7 % (row-major)
+// and 4 % (preshuffled) slower than the skinny rule on average (47 shapes each, us
+// rule / model: 29 x 1328 x 7168 13.6 / 18.1, preshuffled 27 x 4960 x 2560 8.8 /
+// 14.6); the MX families gain (A4W4 1 %, A8W4 4 %).
 #pragma once
 
 namespace aiter_amd {
@@ -86,14 +91,11 @@ inline const GemmCost kGemmCosts[] = {
     {"a16w16_tile_256x256_bplain", 1.59, 0, 3.95, 4.84},
     {"a16w16_tile_96x128_splitk_bplain", 0.345, 0, 6.64, 0.01},
     {"a16w16_tile_64x64_splitk_bplain", 0.237, 0, 5.99, 0.01},
-    {"a16w16_skinny_m32_bplain_lds", 0.0994, 0.105, 0.5, 1.23},
     {"a16w16_tile_128x64_bplain", 0.283, 0, 0.746, 2.8},
     {"a16w16_tile_64x128_bplain", 0.263, 0, 1.77, 1.94},
     {"a16w16_tile_64x64_bplain", 0.22, 0, 3.46, 0.01},
-    {"a16w16_skinny_m32_n32_bplain_lds", 0.04, 0.000485, 3.87, 0.01},
     {"a16w16_skinny_m64_n32_bplain_lds", 0.137, 0.195, 1.53, 0.497},
     {"a16w16_skinny_m64_bplain", 0.246, 0.267, 2.77, 0.01},
-    {"a16w16_skinny_m32_bplain", 0.17, 0.174, 2.14, 0.729},
     {"a16w16_tile_256x256_persist", 1.17, 0, 0.5, 7.59},
     {"a16w16_tile_128x256_persist", 0.694, 0, 0.5, 5.22},
     {"a16w16_tile_128x256", 0.696, 0, 0.5, 6.38},
@@ -110,10 +112,7 @@ inline const GemmCost kGemmCosts[] = {
     {"a16w16_tile_128x128_splitk", 0.49, 0, 5.79, 0.01},
     {"a16w16_tile_64x128_splitk", 0.274, 0, 6.65, 0.01},
     {"a16w16_tile_64x64_splitk", 0.236, 0, 5.82, 0.0154},
-    {"a16w16_skinny_m32", 0.113, 0.000332, 2.45, 0.125},
-    {"a16w16_skinny_m32_n32_alds", 0.0428, 0.0399, 3.64, 0.01},
     {"a16w16_tile_64x64", 0.21, 0, 3.57, 0.01},
-    {"a16w16_skinny_m32_n32", 0.167, 0.189, 0.712, 0.581},
     {"a16w16_skinny_m64_n32_alds", 0.113, 0.185, 1.04, 0.679},
     {"a16w16_skinny_m64", 0.131, 0.195, 2.26, 0.911},
 };

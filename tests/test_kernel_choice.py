@@ -122,3 +122,13 @@ def test_f32_chains_are_no_longer_than_the_simple_rules():
             if "splitk" in choice[0] and "skinny" in choice[0]:
                 continue   # the skinny rule's own split
             assert _chain(choice, k) <= _chain(base, k), (m, n, k, base, choice)
+
+
+def test_bf16_up_to_32_rows_is_the_skinny_rules():
+    log_int = lambda rng, lo, hi, step: max(step, int(math.exp(rng.uniform(math.log(lo), math.log(hi)))) // step * step)
+    rng = random.Random(4)
+    for _ in range(300):
+        m, n, k = rng.randint(1, 32), log_int(rng, 32, 16384, 16), log_int(rng, 512, 28672, 64)
+        for kw in ({"b_pre": False}, {"b_pre": True}, {"b_pre": False, "out_f32": True}):
+            base = gemm_choice("a16w16", m, n, k, splits=1, **kw)[0]
+            assert gemm_choice("a16w16", m, n, k, **kw)[0] == base
