@@ -102,6 +102,7 @@ int tile_splits(int tiles, int stages, int cus) {
 struct ModelScope {
     int batch = 1;
     float margin = 1.06f;     // modelled gain from which another instance replaces the base
+    bool same_form = false;   // a split base gives way to split tiles only, an unsplit one to unsplit ones
     bool persistent = true;   // persistent tiles allowed (no bias, batch or fused epilogue)
 };
 
@@ -218,6 +219,7 @@ const Instance* modelled_choice(const Instance* base, int base_splits, int M, in
     const int chain = base->var.out_f32 ? chain_stages(*base, nst, base_splits) : nst;
     for (const Instance* in : modelled(base->fam, base->var)) {
         if (in->persistent && !sc.persistent) continue;
+        if (sc.same_form && in->split != (base_splits > 1)) continue;
         if (in->skinny && (M > in->bm || M * 2 <= in->bm)) continue;
         if (!in->split) {
             if (chain_stages(*in, nst, 1) > chain) continue;
@@ -566,12 +568,16 @@ Choice choose(const GemmCall& c, int M, int N, int K, bool bias, int cus, Room&&
 
     ModelScope sc;
     sc.batch = c.batch;
-    // a tuned row's tile was the best of all at its own row count: gains
-    // modelled below 8 % measured as ties (bf16 1573 x 14336 x 4096 179.5 us
-    // by the row, 180.1 by the model; 150 x 14336 x 4096 34.7 / 35.2)
-    if (hint) sc.margin = 1.08f;
     sc.persistent = !batched && !bias && !c.epi.kind;
     const int have = batched ? 1 : !inst->split || inst->skinny ? splits : tile_split_count(*inst, M, N, K, cus, splits);
+    // A tuned row's tile was the best of all at its own row count.  Crossing between
+    // split and unsplit forms lost there (us by the row / by the model: bf16 1132 x
+    // 8192 x 28672 545 / 565, A8W4 185 x 8192 x 28672 57 / 67), and among unsplit
+    // tiles modelled gains below 15 % measured -5 to +5 % mostly (bf16 130 to 173 x
+    // 14336 x 4096, modelled 13 %: 0 to -5; A4W4 3136 x 7168 x 2048, 12 %: -12); split
+    // tiles gain what is modelled (bf16 145 x 8192 x 28672 116 / 101, A8W4 170 x
+    // 8192 x 28672 58 / 50).
+    if (hint) sc.same_form = true, sc.margin = have > 1 ? 1.08f : 1.15f;
     const size_t slice = (size_t)M * N * sizeof(float), base_need = have > 1 ? have * slice : 0;
     int sp = 0;
     const Instance* best = modelled_choice(inst, have, M, N, K, cus, sc,

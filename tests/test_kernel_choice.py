@@ -132,3 +132,20 @@ def test_bf16_up_to_32_rows_is_the_skinny_rules():
         for kw in ({"b_pre": False}, {"b_pre": True}, {"b_pre": False, "out_f32": True}):
             base = gemm_choice("a16w16", m, n, k, splits=1, **kw)[0]
             assert gemm_choice("a16w16", m, n, k, **kw)[0] == base
+
+
+@pytest.mark.parametrize("m,n,k,row,splits,keeps", [
+    (1132, 8192, 28672, "a16w16_tile_256x256_bplain_flat", 0, True),    # 545 us, with 4 splits of 256x128 565
+    (150, 14336, 4096, "a16w16_tile_128x128_bplain", 0, True),          # 96x128 within 2 % either way
+    (1275, 4096, 4096, "a16w16_tile_256x128_bplain", 0, False),         # 52.7 us, 160x128 42.7
+    (145, 8192, 28672, "a16w16_tile_256x128_splitk_bplain", 4, False),  # 115.7 us, 160x128 100.6
+])
+def test_what_replaces_a_tuned_rows_tile(m, n, k, row, splits, keeps):
+    """"~row": an unsplit tile gives way to an unsplit one and a split one to a
+    split one, where the model puts it clearly ahead; by its plain name a kernel
+    always runs."""
+    kw = {"b_pre": False, "splits": splits}
+    assert gemm_choice("a16w16", m, n, k, kernel_name=row, **kw)[0] == row
+    choice = gemm_choice("a16w16", m, n, k, kernel_name="~" + row, **kw)
+    assert (choice[0] == row) == keeps
+    assert ("splitk" in choice[0]) == ("splitk" in row)
