@@ -11,12 +11,15 @@
 // out once; traffic: the operands once per tile that reads them.  A split adds
 // its f32 slices at 0.22 us per MB (written, read, summed).
 //
-// The constants are a fit to 8,200 graph-replayed timings under sustained load
-// (977 shapes with 17 to 8192 rows, N 256 to 28672, K 512 to 28672, splits of 2,
-// 4 and 8; weights rotated) on one MI355X.  Against the best instance of each
-// shape the dispatch's choice (modelled_choice(), gemm.hip) is 3.5 % (bf16), 2.5 %
-// (A4W4) and 2 % (A8W4) slower on average; by the simple rule alone it would
-// be 11-12 %, 8 % and 8 %.
+// The constants are fits to graph-replayed timings under sustained load, weights
+// rotated, on one MI355X (17 to 4096 rows, N 256 to 28672, K 512 to 28672, splits
+// of 2, 4 and 8): bf16 9,300 timings over 760 shapes (the forms of a t32 tile for
+// the two weight orders move the same bytes and share theirs), the MX families
+// 4,400 over 600.  Checked on 1,450 shapes, the dispatch's choice (modelled_choice(),
+// gemm.hip) is 3.3 % (bf16), 4.2 % (A4W4) and 2.6 % (A8W4) slower on average than
+// the best instance timed; the simple rule alone is 14 % (row-major bf16), 11 %
+// (preshuffled), 10 % and 8 %.  2 to 5 % of the shapes run over 5 % slower than by
+// the rule.
 //
 // bf16 has no entries up to 32 rows: there the model's choices ran 7 % (row-major)
 // and 4 % (preshuffled) slower than the skinny rule on average (47 shapes each, us
@@ -76,44 +79,44 @@ inline const GemmCost kGemmCosts[] = {
     {"a8w4_skinny_m32_n32", 0.129, 0.25, 1.94, 0.885},
     {"a8w4_tile_32x128", 0.325, 0, 1.53, 2.37},
     {"a8w4_skinny_m64", 0.338, 0.359, 2.35, 0.837},
-    {"a16w16_tile_256x256_bplain_flat", 1.29, 0, 0.5, 8.24},
-    {"a16w16_tile_128x256_bplain", 0.788, 0, 0.5, 5.65},
-    {"a16w16_tile_160x128_bplain", 0.577, 0, 0.632, 3.41},
-    {"a16w16_tile_256x128_bplain", 0.766, 0, 0.5, 5.75},
-    {"a16w16_tile_128x256_splitk_bplain", 0.811, 0, 5.87, 0.01},
-    {"a16w16_tile_128x128_bplain", 0.453, 0, 0.5, 3.44},
-    {"a16w16_tile_256x128_splitk_bplain", 0.796, 0, 4.88, 0.01},
-    {"a16w16_tile_160x128_splitk_bplain", 0.523, 0, 6.44, 0.01},
-    {"a16w16_tile_64x128_splitk_bplain", 0.279, 0, 6.63, 0.01},
-    {"a16w16_tile_96x128_bplain", 0.245, 0, 6.02, 0.01},
-    {"a16w16_tile_128x64_splitk_bplain", 0.36, 0, 4.01, 1},
-    {"a16w16_tile_128x128_splitk_bplain", 0.487, 0, 5.87, 0.01},
-    {"a16w16_tile_256x256_bplain", 1.59, 0, 3.95, 4.84},
-    {"a16w16_tile_96x128_splitk_bplain", 0.345, 0, 6.64, 0.01},
-    {"a16w16_tile_64x64_splitk_bplain", 0.237, 0, 5.99, 0.01},
-    {"a16w16_tile_128x64_bplain", 0.283, 0, 0.746, 2.8},
-    {"a16w16_tile_64x128_bplain", 0.263, 0, 1.77, 1.94},
-    {"a16w16_tile_64x64_bplain", 0.22, 0, 3.46, 0.01},
-    {"a16w16_skinny_m64_n32_bplain_lds", 0.137, 0.195, 1.53, 0.497},
+    {"a16w16_tile_256x256_bplain_flat", 1.34, 0, 0.5, 6.97},
+    {"a16w16_tile_128x256_bplain", 0.821, 0, 0.5, 4.73},
+    {"a16w16_tile_160x128_bplain", 0.56, 0, 0.5, 3.61},
+    {"a16w16_tile_256x128_bplain", 0.761, 0, 0.5, 4.76},
+    {"a16w16_tile_128x256_splitk_bplain", 0.814, 0, 6.87, 0.01},
+    {"a16w16_tile_128x128_bplain", 0.469, 0, 0.5, 2.93},
+    {"a16w16_tile_256x128_splitk_bplain", 0.759, 0, 4.82, 2.02},
+    {"a16w16_tile_160x128_splitk_bplain", 0.542, 0, 6.59, 0.01},
+    {"a16w16_tile_64x128_splitk_bplain", 0.375, 0, 5.4, 0.177},
+    {"a16w16_tile_96x128_bplain", 0.417, 0, 0.5, 2.35},
+    {"a16w16_tile_128x64_splitk_bplain", 0.349, 0, 3.18, 1.99},
+    {"a16w16_tile_128x128_splitk_bplain", 0.483, 0, 6.22, 0.01},
+    {"a16w16_tile_256x256_bplain", 1.68, 0, 1.4, 5.43},
+    {"a16w16_tile_96x128_splitk_bplain", 0.436, 0, 5.73, 0.01},
+    {"a16w16_tile_64x64_splitk_bplain", 0.237, 0, 5.87, 0.01},
+    {"a16w16_tile_128x64_bplain", 0.309, 0, 0.561, 2.26},
+    {"a16w16_tile_64x128_bplain", 0.331, 0, 0.5, 2.16},
+    {"a16w16_tile_64x64_bplain", 0.244, 0, 2.26, 0.435},
+    {"a16w16_skinny_m64_n32_bplain_lds", 0.137, 0.215, 1.44, 0.523},
     {"a16w16_skinny_m64_bplain", 0.246, 0.267, 2.77, 0.01},
-    {"a16w16_tile_256x256_persist", 1.17, 0, 0.5, 7.59},
-    {"a16w16_tile_128x256_persist", 0.694, 0, 0.5, 5.22},
-    {"a16w16_tile_128x256", 0.696, 0, 0.5, 6.38},
-    {"a16w16_tile_160x128", 0.583, 0, 1.22, 2.65},
-    {"a16w16_tile_256x128", 0.742, 0, 0.5, 5.81},
-    {"a16w16_tile_256x256", 1.2, 0, 0.5, 9.78},
-    {"a16w16_tile_128x128", 0.455, 0, 0.798, 3.26},
-    {"a16w16_tile_160x128_splitk", 0.583, 0, 5.53, 0.01},
-    {"a16w16_tile_96x128", 0.391, 0, 0.625, 2.44},
-    {"a16w16_tile_96x128_splitk", 0.395, 0, 5.91, 0.01},
-    {"a16w16_tile_64x128", 0.262, 0, 1.19, 2.45},
-    {"a16w16_tile_128x64_splitk", 0.354, 0, 4.22, 0.931},
-    {"a16w16_tile_128x64", 0.275, 0, 0.617, 2.96},
-    {"a16w16_tile_128x128_splitk", 0.49, 0, 5.79, 0.01},
-    {"a16w16_tile_64x128_splitk", 0.274, 0, 6.65, 0.01},
-    {"a16w16_tile_64x64_splitk", 0.236, 0, 5.82, 0.0154},
-    {"a16w16_tile_64x64", 0.21, 0, 3.57, 0.01},
-    {"a16w16_skinny_m64_n32_alds", 0.113, 0.185, 1.04, 0.679},
+    {"a16w16_tile_256x256_persist", 1.26, 0, 0.5, 5.94},
+    {"a16w16_tile_128x256_persist", 0.753, 0, 0.5, 3.65},
+    {"a16w16_tile_128x256", 0.759, 0, 0.5, 4.49},
+    {"a16w16_tile_160x128", 0.56, 0, 0.5, 3.61},
+    {"a16w16_tile_256x128", 0.761, 0, 0.5, 4.76},
+    {"a16w16_tile_256x256", 1.26, 0, 0.5, 7.98},
+    {"a16w16_tile_128x128", 0.469, 0, 0.5, 2.93},
+    {"a16w16_tile_160x128_splitk", 0.542, 0, 6.59, 0.01},
+    {"a16w16_tile_96x128", 0.417, 0, 0.5, 2.35},
+    {"a16w16_tile_96x128_splitk", 0.436, 0, 5.73, 0.01},
+    {"a16w16_tile_64x128", 0.331, 0, 0.5, 2.16},
+    {"a16w16_tile_128x64_splitk", 0.349, 0, 3.18, 1.99},
+    {"a16w16_tile_128x64", 0.309, 0, 0.561, 2.26},
+    {"a16w16_tile_128x128_splitk", 0.483, 0, 6.22, 0.01},
+    {"a16w16_tile_64x128_splitk", 0.375, 0, 5.4, 0.177},
+    {"a16w16_tile_64x64_splitk", 0.237, 0, 5.87, 0.01},
+    {"a16w16_tile_64x64", 0.244, 0, 2.26, 0.435},
+    {"a16w16_skinny_m64_n32_alds", 0.113, 0.192, 1.43, 0.503},
     {"a16w16_skinny_m64", 0.131, 0.195, 2.26, 0.911},
 };
 
