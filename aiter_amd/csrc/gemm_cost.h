@@ -15,7 +15,7 @@
 // rotated, on one MI355X (17 to 4096 rows, N 256 to 28672, K 512 to 28672, splits
 // of 2, 4 and 8): bf16 9,300 timings over 760 shapes (the forms of a t32 tile for
 // the two weight orders move the same bytes and share theirs), the MX families
-// 4,400 over 600.  Checked on 1,450 shapes, the dispatch's choice (modelled_choice(),
+// an earlier 8,200 over 977 shapes of all families.  Checked on 1,450 shapes, the dispatch's choice (modelled_choice(),
 // gemm.hip) is 3.3 % (bf16), 4.2 % (A4W4) and 2.6 % (A8W4) slower on average than
 // the best instance timed; the simple rule alone is 14 % (row-major bf16), 11 %
 // (preshuffled), 10 % and 8 %.  2 to 5 % of the shapes run over 5 % slower than by
