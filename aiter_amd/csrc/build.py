@@ -83,17 +83,18 @@ def _compile_binding(out_dir: str) -> str:
     return obj
 
 
-def _link_binding(obj: str) -> None:
+def _link_binding(obj: str, out_dir: str) -> str:
+    """Against the library in ``out_dir``."""
     import torch
 
-    tmp = NATIVE + ".tmp"
-    cmd = [os.environ.get("CXX", "g++"), "-shared", "-fPIC", "-o", tmp, obj, "-L" + PKG, "-l:libaiter_amd.so",
+    tmp = os.path.join(out_dir, os.path.basename(NATIVE))
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-fPIC", "-o", tmp, obj, "-L" + out_dir, "-l:libaiter_amd.so",
            "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
            "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"_native.so does not link:\n{r.stderr[-4000:]}")
-    os.replace(tmp, NATIVE)
+    return tmp
 
 
 def build(verbose: bool = True) -> str:
@@ -107,13 +108,15 @@ def build(verbose: bool = True) -> str:
     with open(os.path.join(out_dir, "vgpr_spills.txt"), "w") as f:
         for k, v in sorted(spills.items()):
             f.write(f"{v}\t{k}\n")
-    tmp = LIB + ".tmp"
+    tmp = os.path.join(out_dir, os.path.basename(LIB))
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
+    native = _link_binding(binding.result(), out_dir)
+    # both at the end: a failed build leaves the pair that was there
     os.replace(tmp, LIB)
-    _link_binding(binding.result())
+    os.replace(native, NATIVE)
     if verbose:
         print(f"built {LIB}")
         if spills:
