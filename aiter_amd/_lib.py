@@ -155,6 +155,10 @@ SIGNATURES = {
 }
 
 
+def _minor(version: str) -> list:
+    return version.split("+")[0].split(".")[:2]
+
+
 def lib():
     """Load the in-tree library (raises if it is missing: there is no fallback)."""
     global _lib
@@ -178,6 +182,11 @@ def lib():
             except ImportError as e:
                 raise RuntimeError(f"aiter_amd/_native.so is not built for this Python and torch ({e}); "
                                    "run `python -m aiter_amd.csrc.build`") from e
+            # it reads torch's C++ objects, whose layout holds within a minor version
+            built = getattr(native, "torch_version", "an unknown version")
+            if _minor(built) != _minor(torch.__version__):
+                raise RuntimeError(f"aiter_amd/_native.so is built for torch {built}, this is "
+                                   f"{torch.__version__}; run `python -m aiter_amd.csrc.build`")
             _native.update({n: getattr(native, n) for n in SIGNATURES if hasattr(native, n)})
             _lib = l
     return _lib

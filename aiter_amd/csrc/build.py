@@ -66,12 +66,18 @@ def _compile(src: str, out_dir: str, extra=()) -> tuple:
     return obj, vgpr_spills(r.stderr)
 
 
+def binding_defines(torch) -> list:
+    """Macros of binding.cpp: the torch it is built against."""
+    return [f'-DAITER_AMD_TORCH="{torch.__version__}"']
+
+
 def _compile_binding(out_dir: str) -> str:
     import torch
 
     inc = os.path.join(os.path.dirname(torch.__file__), "include")
     obj = os.path.join(out_dir, "binding.o")
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           *binding_defines(torch),
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", inc, "-isystem",
            os.path.join(inc, "torch", "csrc", "api", "include"), "-isystem",
            os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), "-isystem",

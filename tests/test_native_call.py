@@ -57,3 +57,23 @@ def test_missing_native_module_raises(monkeypatch):
     monkeypatch.setattr(_lib.importlib, "import_module", missing)
     with pytest.raises(RuntimeError, match="_native.so is not built"):
         _lib.lib()
+
+
+@pytest.mark.parametrize("version,ok", [(torch.__version__, True), ("1.2.3+rocm7.0", False)])
+def test_module_of_another_torch_raises(version, ok, monkeypatch):
+    """The module reads torch's C++ objects: one that was compiled for another
+    minor version is refused."""
+    _lib.lib()
+    real = _lib.importlib.import_module("aiter_amd._native")
+    assert real.torch_version == torch.__version__
+
+    class Other:
+        torch_version = version
+
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib.importlib, "import_module", lambda name: Other)
+    if ok:
+        _lib.lib()
+    else:
+        with pytest.raises(RuntimeError, match="built for torch 1.2.3"):
+            _lib.lib()
