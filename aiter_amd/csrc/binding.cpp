@@ -40,8 +40,12 @@ int dtype_id(at::ScalarType t) {
         case at::kLong: return AITER_DTYPE_i64;
         case at::kUInt64: return AITER_DTYPE_u64;
         case at::kFloat8_e4m3fn: return AITER_DTYPE_fp8;
+#if AITER_AMD_TORCH_E8M0
         case at::kFloat8_e8m0fnu: return AITER_DTYPE_fp8_e8m0;
+#endif
+#if AITER_AMD_TORCH_FP4
         case at::kFloat4_e2m1fn_x2: return AITER_DTYPE_fp4x2;
+#endif
         default: return -1;
     }
 }

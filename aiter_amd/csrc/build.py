@@ -67,8 +67,11 @@ def _compile(src: str, out_dir: str, extra=()) -> tuple:
 
 
 def binding_defines(torch) -> list:
-    """Macros of binding.cpp: the torch it is built against."""
-    return [f'-DAITER_AMD_TORCH="{torch.__version__}"']
+    """Macros of binding.cpp: the torch it is built against, and which of the
+    newer element types that torch has."""
+    return [f'-DAITER_AMD_TORCH="{torch.__version__}"',
+            f"-DAITER_AMD_TORCH_E8M0={int(hasattr(torch, 'float8_e8m0fnu'))}",
+            f"-DAITER_AMD_TORCH_FP4={int(hasattr(torch, 'float4_e2m1fn_x2'))}"]
 
 
 def _compile_binding(out_dir: str) -> str:

@@ -32,3 +32,14 @@ def test_failed_binding_keeps_the_built_pair(step, tmp_path, monkeypatch):
     with pytest.raises(RuntimeError):
         build.build(verbose=False)
     assert open(build.LIB).read() == open(build.NATIVE).read() == "before"
+
+
+def test_binding_for_a_torch_without_the_newer_types(tmp_path):
+    """The element types that the Python side takes only where torch has them
+    are optional in the native caller too."""
+    old = types.SimpleNamespace(__version__="2.6.0")
+    assert build.binding_defines(old)[1:] == ["-DAITER_AMD_TORCH_E8M0=0", "-DAITER_AMD_TORCH_FP4=0"]
+    text = open(os.path.join(build.HERE, "binding.cpp")).read()
+    for name, macro in (("kFloat8_e8m0fnu", "AITER_AMD_TORCH_E8M0"), ("kFloat4_e2m1fn_x2", "AITER_AMD_TORCH_FP4")):
+        assert [part.split("#endif")[0].count(name) for part in text.split(f"#if {macro}\n")[1:]] == [1]
+        assert text.count(name) == 1
