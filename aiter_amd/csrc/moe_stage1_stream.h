@@ -5,7 +5,7 @@
 // keeps one K stage per workgroup ahead and meets at a barrier per stage; here
 // each wave has 8 KB of weights in flight and none to wait for.
 #pragma once
-#include <cmath>
+#include <algorithm>
 
 #include "gemm_flat.h"
 
@@ -23,14 +23,14 @@ struct S1Ops {
 // registers, one 256-element window ahead, with no barrier until its sums are
 // added through LDS in wave order.
 template <int NWK, int C>
-AA_DEV void stage1_stream_body(const GemmParams& p, const MoeParams& mq, f32x4_t (*part)[4][64]) {
+AA_DEV void stage1_stream_body(const GemmParams& p, const MoeParams& mq, int units, int block,
+                               f32x4_t (*part)[4][64]) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kpart = wave % NWK;
     const int cols = mq.inter / 32;
-    const int item = blockIdx.x * (8 / NWK) + wave / NWK;
+    const int item = block * (8 / NWK) + wave / NWK;
     const int u = item / cols, cg = item % cols;
-    const int units = min((mq.num_valid[0] + 31) / 32, (mq.sorted_len + 31) / 32);
     const int pos0 = 32 * u;
 
     const bool in = u < units && pos0 + (lane & 31) < mq.sorted_len;
@@ -160,35 +160,44 @@ AA_DEV void stage1_stream_body(const GemmParams& p, const MoeParams& mq, f32x4_t
     if (lane < 16) mq.q_scale[mx::scale_shuffle_idx(mq.q_scale_n_pad, pos, cg)] = (uint8_t)byte;
 }
 
-template <int NWK>
-__global__ __launch_bounds__(512, 4) void moe_stage1_stream_kernel(GemmParams p, MoeParams mq) {
-    __shared__ f32x4_t part[NWK > 1 ? 8 : 1][4][64];
-    if (blockIdx.y == 0) stage1_stream_body<NWK, 0>(p, mq, part);
-    else stage1_stream_body<NWK, 1>(p, mq, part);
+// Waves per item: the most (up to 8) whose items fit `waves`, 8 per CU: where some
+// CUs have two workgroups those end last (257 experts, 7168 x 2 * 256: 32 tokens
+// 57.3 us with 1 wave per item, 70.0 with 2, 63.4 with 4).  The items are those of
+// the units that hold rows, which only the sort knows: routing may be uneven (64
+// tokens on 18 experts 19.9 us; 91 with the waves that even routing would
+// leave, 30 by the flat kernel).
+template <int C>
+AA_DEV void stage1_stream_part(const GemmParams& p, const MoeParams& mq, int waves, int units,
+                               f32x4_t (*part)[4][64]) {
+    const int items = units * (mq.inter / 32), block = blockIdx.x;
+    if (items * 8 <= waves) stage1_stream_body<8, C>(p, mq, units, block, part);
+    else if (items * 4 <= waves) stage1_stream_body<4, C>(p, mq, units, block, part);
+    else if (items * 2 <= waves) stage1_stream_body<2, C>(p, mq, units, block, part);
+    else stage1_stream_body<1, C>(p, mq, units, block, part);
 }
 
-// The items of the experts that `entries` routed rows are expected to touch
-inline double stage1_stream_items(const MoeParams& mq, int64_t entries) {
-    return mq.n_experts * (1.0 - std::exp(-(double)entries / mq.n_experts)) * (mq.inter / 32);
+// blockIdx.y 0: first halves; 1: second halves likewise, or 1 to 8: second halves
+// with 8 waves per item
+__global__ __launch_bounds__(512, 4) void moe_stage1_stream_kernel(GemmParams p, MoeParams mq, int waves) {
+    __shared__ f32x4_t part[8][4][64];
+    const int units = __builtin_amdgcn_readfirstlane(min((mq.num_valid[0] + 31) / 32, (mq.sorted_len + 31) / 32));
+    if (blockIdx.y == 0) stage1_stream_part<0>(p, mq, waves, units, part);
+    else if (gridDim.y == 2) stage1_stream_part<1>(p, mq, waves, units, part);
+    else stage1_stream_body<8, 1>(p, mq, units, (blockIdx.y - 1) * gridDim.x + blockIdx.x, part);
 }
 
-// Waves per item: the most (up to 8) that keep one workgroup of 8 waves per CU;
-// where some CUs have two, those end last (32 tokens at the shape below: 57.3
-// us with 1 wave per item, 70.0 with 2, 63.4 with 4).
+// `units`: the most that can hold rows.  The grid has room for one wave of each of
+// their items, or for all the waves that the CUs take one workgroup of.
 inline void launch_stage1_stream(const GemmParams& p, const MoeParams& mq, int64_t units, int64_t entries, int cus,
                                  hipStream_t st) {
-    const double items = stage1_stream_items(mq, entries);
-    int nwk = 1;
-    while (nwk < 8 && items * nwk * 2 <= 8.0 * cus) nwk *= 2;
-    const int64_t wgs = (units * (mq.inter / 32) * nwk + 7) / 8;
-    // up to 16 entries fill no second half of a unit
-    const dim3 grid((unsigned)wgs, entries > 16 ? 2 : 1);
-    switch (nwk) {
-        case 1: moe_stage1_stream_kernel<1><<<grid, 512, 0, st>>>(p, mq); break;
-        case 2: moe_stage1_stream_kernel<2><<<grid, 512, 0, st>>>(p, mq); break;
-        case 4: moe_stage1_stream_kernel<4><<<grid, 512, 0, st>>>(p, mq); break;
-        default: moe_stage1_stream_kernel<8><<<grid, 512, 0, st>>>(p, mq); break;
-    }
+    const int64_t items = units * (mq.inter / 32);
+    const int64_t wgs = std::max((items + 7) / 8, std::min<int64_t>(items, cus));
+    // Up to 16 entries fill no second half of a unit, up to 16 tokens hardly any.
+    // Above, a few experts with more rows than that are usual, and one workgroup
+    // that walks such a half's whole K beside a first half on its CU ends last (64
+    // tokens, one expert with 17 rows: 95 us, with 8 waves per item 68).
+    const dim3 grid((unsigned)wgs, entries <= 16 ? 1 : mq.token_num <= 16 ? 2 : 9);
+    moe_stage1_stream_kernel<<<grid, 512, 0, st>>>(p, mq, 8 * (int)std::min<int64_t>(wgs, cus));
 }
 
 }  // namespace aiter_amd

@@ -424,12 +424,14 @@ def _stream_stage1(token_num: int, topk: int, experts: int) -> bool:
     """Stage 1 on the weight-streaming kernel: up to 3 routed rows per expert.
 
     us per launch, flat kernel / streaming kernel (experts, topk, model_dim,
-    inter_dim; tokens): 257, 9, 7168, 256: 10.9 / 9.5 at 1, 31.6 / 22.3 at 8,
-    85 / 67 at 64 (2.2 rows per expert), 93 / 104 at 100 (3.5); 256, 8, 3072,
-    256: 22.3 / 19.0 at 16, 49 / 34 at 100 (3.1), 45.6 / 47.6 at 128 (4); 128,
-    8, 4096, 512: 19.0 / 14.1 at 4, 53 / 41 at 48 (3), 58 / 65 at 100 (6.3).
-    Past that an item's 16-row halves both hold rows and its weights are read
-    by two waves, where the flat kernel shares them through LDS."""
+    inter_dim; tokens), scores of near-even popularity: 257, 9, 7168, 256: 10.0
+    / 9.3 at 1, 27.4 / 21.1 at 8, 84 / 68 at 64; 256, 8, 3072, 256: 22.4 / 18.2 at
+    16, 37 / 32 at 85; 128, 8, 4096, 512: 19.2 / 14.7 at 4, 47 / 41 at 48; uneven
+    ones (some experts with half of the tokens): 66 / 43, 35 / 23 and 46 / 34 at
+    the last of each.  Past the line the flat kernel's shared B tiles catch up: at
+    4 rows per expert 96 / 79, 39 / 37 and 53 / 48, level at 5 to 8 (256, 8, 3072,
+    256: 39.4 / 39.3 at 5), behind at 12 (99 / 126, 43 / 56, 59 / 71).  The line is on
+    the safe side of that."""
     return token_num * topk <= STREAM_ROWS_PER_EXPERT * experts
 
 

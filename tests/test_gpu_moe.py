@@ -564,6 +564,21 @@ def test_stage1_stream(cuda, m, e, topk, dim, inter, bs, act, doweight):
     assert np.mean(got != ref) < 0.005
 
 
+@pytest.mark.parametrize("m,e,topk,hot,dim", [(64, 257, 9, 18, 1536), (16, 257, 9, 9, 1536), (17, 64, 4, 4, 1024),
+                                              (40, 40, 3, 8, 2304), (85, 257, 9, 257, 768)])
+def test_stage1_stream_uneven_routing(cuda, m, e, topk, hot, dim, monkeypatch):
+    """All tokens on `hot` experts: fewer units hold rows than the launch has room
+    for, so more waves share an item's K, and both halves of most units have rows
+    (16 and 17 tokens: the two ways second halves are launched)."""
+    def routing(m, e, topk, rng):
+        ids = np.stack([rng.choice(hot, topk, replace=False) for _ in range(m)]).astype(np.int32) * (e // hot)
+        w = rng.random((m, topk)).astype(np.float32) + 0.05
+        return ids, (w / w.sum(1, keepdims=True)).astype(np.float32)
+
+    monkeypatch.setattr(sys.modules[__name__], "_routing", routing)
+    test_stage1_stream(cuda, m, e, topk, dim, 256, 32, 0, False)
+
+
 @pytest.mark.parametrize("m", [1, 33, 64, 65, 128])
 @pytest.mark.parametrize("dim,inter", [(512, 256), (512, 512), (6144, 256), (6400, 512)])
 def test_stage2_reduce(cuda, m, dim, inter):
