@@ -99,9 +99,9 @@ def row_kernel(row: TunedRow, m: int) -> str:
     """The row's kernel name as the library takes it for ``m`` rows.  From 64
     rows on, a shipped row tuned at 1.25 times the rows or more (the
     power-of-two padding of the lookup) names a tile that may leave a good part
-    of itself empty: "~name" lets the library's time model replace it (bf16 1200 x
-    4096 x 4096, tuned at 2048 rows: 51.9 us by the row, 43.1 by the model's
-    160x128 tile; A4W4 2500 x 7168 x 2048 32.2 and 28.2)."""
+    of itself empty: "~name" lets the library's time model replace it (bf16 1208 x
+    4096 x 4096, tuned at 2048 rows: 50.4 us by the row, 41.8 by the model's
+    160x128 tile; A4W4 2484 x 7168 x 2048 29.7 and 28.0)."""
     name = str(row.get("kernelName", "") or "")
     return "~" + name if name and row.rows > 64 and row.rows >= 1.25 * m else name
 

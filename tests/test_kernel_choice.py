@@ -9,7 +9,7 @@ import pandas as pd
 import pytest
 import torch
 
-from aiter_amd import fused_gemm, gemm_op_a4w4, tuner
+from aiter_amd import config, fused_gemm, gemm_op_a4w4, gemm_op_a8w4, tuned_gemm, tuner
 from aiter_amd._lib import gemm_choice, instance_table, kernel_names, kernel_table
 from aiter_amd.csrc import build
 from tests.test_dispatch import _clear, _row, gfx950  # noqa: F401
@@ -178,3 +178,80 @@ def test_cost_table_is_plausible():
         twin = (*a[:2], False, *a[3:])
         if a[2] and twin in costs and not (a[3] >= 128 and a[4] == 256):
             assert 0.8 <= ta / costs[twin] <= 1.25, (a, ta, costs[twin])
+
+
+TABLES = {"a4w4": ("AITER_CONFIG_GEMM_A4W4", gemm_op_a4w4.get_GEMM_config),
+          "a8w4": ("AITER_CONFIG_GEMM_A8W4", gemm_op_a8w4.get_GEMM_A8W4_config),
+          "a16w16": ("AITER_CONFIG_GEMM_BF16", lambda m, n, k: tuned_gemm.get_GEMM_A16W16_config(
+              m, n, k, False, "torch.bfloat16", "torch.bfloat16"))}
+
+
+def _table(fam, rows):
+    """a tuned CSV of the family with (M, N, K, kernel) rows"""
+    extra = {"bias": False, "dtype": "torch.bfloat16", "outdtype": "torch.bfloat16", "scaleAB": False,
+             "bpreshuffle": False, "libtype": "aiter_amd", "solidx": 1} if fam == "a16w16" else {}
+    return pd.DataFrame([{**_row(m, n, k, name), **extra} for m, n, k, name in rows])
+
+
+@pytest.mark.parametrize("fam", TABLES)
+@pytest.mark.parametrize("shipped", [True, False])
+def test_rows_tuned_for_other_row_counts(fam, shipped, tmp_path, monkeypatch, gfx950):
+    """A shipped row above 64 rows that serves a call of 1/1.25 of its rows or
+    fewer is handed on as "~name"; a row of the caller's own list by its name."""
+    name = f"{fam}_tile_128x128" + ("_bplain" if fam == "a16w16" else "")
+    path = tmp_path / "t.csv"
+    _table(fam, [(512, 512, 512, name), (64, 512, 512, name)]).to_csv(path, index=False)
+    env, lookup = TABLES[fam]
+    if shipped:
+        monkeypatch.delenv(env, raising=False)
+        for mod in (gemm_op_a4w4, gemm_op_a8w4, tuned_gemm):
+            for const in ("DEFAULT_A4W4_CSV", "DEFAULT_A8W4_CSV", "DEFAULT_BF16_CSV"):
+                if hasattr(mod, const):
+                    monkeypatch.setattr(mod, const, str(path))
+    else:
+        monkeypatch.setenv(env, str(path))
+    _clear()
+    for m, rows in ((512, 512), (410, 512), (409, 512), (257, 512), (64, 64), (33, 64)):
+        row = lookup(m, 512, 512)
+        assert row["kernelName"] == name and row.rows == (rows if shipped else m)
+        assert config.row_kernel(row, m) == ("~" if shipped and rows == 512 and m <= 409 else "") + name
+
+
+@pytest.mark.parametrize("shipped", [True, False])
+def test_the_call_takes_the_hint(shipped, tmp_path, monkeypatch, gfx950):
+    """The three entries pass the row's kernel on as row_kernel writes it."""
+    m, mark, seen = 300, "~" if shipped else "", []
+    for fam, mod in (("a4w4", gemm_op_a4w4), ("a8w4", gemm_op_a8w4), ("a16w16", tuned_gemm)):
+        name = f"{fam}_tile_128x128" + ("_bplain" if fam == "a16w16" else "")
+        path = tmp_path / f"{fam}.csv"
+        _table(fam, [(512, 512, 512, name)]).to_csv(path, index=False)
+        if shipped:
+            monkeypatch.delenv(TABLES[fam][0], raising=False)
+            const = {"a4w4": "DEFAULT_A4W4_CSV", "a8w4": "DEFAULT_A8W4_CSV", "a16w16": "DEFAULT_BF16_CSV"}[fam]
+            monkeypatch.setattr(mod, const, str(path))
+        else:
+            monkeypatch.setenv(TABLES[fam][0], str(path))
+        monkeypatch.setattr(mod, "call", lambda *a: seen.append(a))
+    _clear()
+    u8 = lambda r, c: torch.zeros(r, c, dtype=torch.uint8)
+    gemm_op_a4w4.gemm_a4w4(u8(m, 256), u8(512, 256), u8(512, 16), u8(512, 16))
+    gemm_op_a8w4.gemm_a8w4_mxfp8(u8(m, 512), u8(512, 256), u8(512, 16), u8(512, 16), a_preshuffle=False)
+    tuned_gemm.tgemm.mm(torch.zeros(m, 512, dtype=torch.bfloat16), torch.zeros(512, 512, dtype=torch.bfloat16))
+    assert [next(x for x in a[1:] if isinstance(x, str)) for a in seen] == [
+        mark + "a4w4_tile_128x128", mark + "a8w4_tile_128x128", mark + "a16w16_tile_128x128_bplain"]
+
+
+@pytest.mark.parametrize("fam,m,n,k,kw,choice", [
+    ("a4w4", 43, 4096, 4096, {}, "a4w4_skinny_m64_n32_alds"), ("a4w4", 150, 14336, 4096, {}, "a4w4_tile_96x128"),
+    ("a8w4", 300, 7168, 16384, {}, "a8w4_tile_96x128"),
+    ("a16w16", 600, 7168, 2048, {"b_pre": False}, "a16w16_tile_160x128_bplain"),
+    ("a16w16", 150, 4096, 14336, {"b_pre": False}, "a16w16_tile_160x128_splitk_bplain"),
+    ("a16w16", 4001, 4096, 14336, {"b_pre": False}, "a16w16_tile_256x256_bplain_flat"),
+])
+def test_instance_chosen(fam, m, n, k, kw, choice):
+    """Calls whose choice is not the simple rule's tile, by instance; with a
+    split request or a kernel named the model has no say."""
+    base = gemm_choice(fam, m, n, k, splits=1, **kw)[0]
+    got = gemm_choice(fam, m, n, k, **kw)[0]
+    assert got == choice != base
+    assert gemm_choice(fam, m, n, k, kernel_name=base, **kw)[0] == base
