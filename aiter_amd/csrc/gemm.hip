@@ -563,7 +563,8 @@ Choice choose(const GemmCall& c, int M, int N, int K, bool bias, int cus, Room&&
     }
     if (!inst->split) splits = 1;
     else if (req_splits > 0) splits = req_splits;
-    else if (!inst->skinny) splits = tile_splits(((M + inst->bm - 1) / inst->bm) * ((N + inst->bn - 1) / inst->bn), nst, cus);
+    else if (!inst->skinny)
+        splits = tile_splits(((M + inst->bm - 1) / inst->bm) * ((N + inst->bn - 1) / inst->bn), nst, cus);
     if (!(hint || (!named && req_splits == 0)) || M <= 16 || !inst->cost) return {inst, splits};
 
     ModelScope sc;
